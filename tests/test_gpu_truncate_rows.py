@@ -1,0 +1,58 @@
+"""GPU: truncation statistics of rows that start anywhere in a 16-byte line, end inside a tile of the streaming pass
+(8192 elements, segments of tiles 0 mod 16, 4 mod 16, 2 mod 4 and the odd ones), or keep their likely tokens where
+the pass sees them last; against the fp64 oracle."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import accept as A
+from trida_stack_amd import kernels as TK
+
+pytestmark = pytest.mark.gpu
+
+TILE = 8192
+
+
+def check(x, T, k, p, ban=-1):
+    """x: fp32 rows [B, R, V] on the GPU, any strides. The kept set matches but for a boundary within 1e-6 of top_p;
+    the normaliser to 1e-6 (the 24-bit exponentials of the histogram)."""
+    m, thr, zk, st, _ = (t.cpu().numpy() for t in TK.truncate_stats(x, temperature=T, top_k=k, top_p=p, ban_id=ban,
+                                                                    want_passes=True))
+    logits = x.cpu().numpy()
+    _, info = A.truncated_probs(logits, T, k, p, ban, return_info=True)
+    y = logits.copy()
+    if ban >= 0:
+        y[..., ban] = -np.inf
+    y = (y / np.float32(T)).astype(np.float32).astype(np.float64)
+    assert (st == 0).all() and (m == y.max(-1).astype(np.float32)).all()
+    for at in np.ndindex(m.shape):
+        if info.boundary_gap[at] < 1e-6:
+            continue
+        kept = info.kept[at] & np.isfinite(y[at])
+        assert (kept == (np.isfinite(y[at]) & (y[at] >= thr[at]))).all(), (at, kept.sum())
+        z = np.exp(y[at][kept] - y[at].max()).sum()
+        assert abs(zk[at] / z - 1) < 1e-6, (at, zk[at], z)
+
+
+@pytest.mark.parametrize("V", [1, 3, 7, 2051, TILE - 1, TILE + 1, 2 * TILE + 6, 5 * TILE - 3, 17 * TILE + 2])
+@pytest.mark.parametrize("T,k,p", [(0.7, 0, 0.95), (1.0, 20, 0.9), (1.2, 0, 1.0)])
+def test_unaligned_rows(gpu, V, T, k, p):
+    g = torch.Generator(device=gpu).manual_seed(V)
+    buf = torch.randn(4 * (V + 5), generator=g, device=gpu) * 3
+    x = buf[1: 1 + 4 * (V + 1)].view(1, 4, V + 1)[..., :V]  # rows at every offset within a line, for odd V + 1
+    check(x, T, k, p, ban=V // 2 if V > 1 else -1)
+
+
+@pytest.mark.parametrize("T,k,p", [(0.7, 0, 0.95), (0.5, 0, 0.8), (1.2, 0, 0.98), (1.0, 50, 0.95), (1.0, 0, 1.0)])
+def test_late_tokens(gpu, T, k, p):
+    """Likely tokens in the last segment only, the first one only, a vocabulary sorted by frequency, a row whose
+    whole mass is one token, and one with more values in the boundary bin than are ranked against each other."""
+    V, g = 20 * TILE + 5, torch.Generator(device=gpu).manual_seed(3)
+    x = torch.randn(6, V, generator=g, device=gpu) * 2
+    x[0, 19 * TILE: 19 * TILE + 20] += 14 * torch.rand(20, generator=g, device=gpu)
+    x[1, 5: 25] += 14 * torch.rand(20, generator=g, device=gpu)
+    x[2] = x[2].sort(descending=True).values
+    x[3, 3 * TILE + 7] = 25.0
+    x[4] = x[4].mul(8).round().div(8)   # massive ties
+    x[5] = x[5].mul(0.05)               # a flat row: everything within a few bins
+    check(x.view(2, 3, V), T, k, p)

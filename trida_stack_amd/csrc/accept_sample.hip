@@ -4,12 +4,19 @@
 //   truncate (grid rows): one 512-thread block per verify row finds the truncated distribution's
 //       statistics: m = max y (y = logit / T, the banned id at -inf), thr = the smallest kept y and
 //       Zk = sum over kept y of exp(y - m), so that P(x) = [y_x >= thr] exp(y_x - m) / Zk.
-//       A sorted, evenly spaced 2048-element sample of the row places a window that should hold the
-//       truncation boundary; ONE streaming pass then accumulates the row max, the total mass, the mass
-//       above the window, and collects the window's values into LDS, where a bitonic sort and an fp64
-//       prefix scan resolve thr exactly. When the window misses (a few heavy tokens outside the
-//       sample, massive ties, |y| large enough to overflow the sample-relative exponentials) the block
-//       falls back to an exact radix select over the order-preserving keys of y, 8 bits per pass.
+//       An evenly spaced 2048-element sample of the row places a window that should hold the truncation
+//       boundary; ONE streaming pass, in four segments spread over the row, then accumulates the row max, a
+//       histogram of the values that can matter (the mass of the others, most of the row, stays in
+//       registers) and collects the window's values into LDS, the window being placed anew from the
+//       histogram after each segment. The boundary bin's values settle thr exactly. Segments whose window
+//       missed are streamed again; rows out of the histogram's range (massive ties, |y| large enough to overflow
+//       the sample-relative exponentials) take an exact radix select over the order-preserving keys of
+//       y, 8 bits per pass.
+//       Bound by the instructions of 16 waves per CU beside the row's bytes (two rows per CU at a time). 512
+//       rows of 248320, half of them peaked: 290 -> 189 us at T = 0.7, top_p = 0.95 (478 -> 123 at 0.5 / 0.8,
+//       259 -> 269 at 1.2 / 0.98, where two thirds of a row are kept and the boundary moves with each late
+//       token), 230 -> 122 with top_k = 50, 118 -> 96 (5.3 TB/s) untruncated; rows of 248319, which scalar loads
+//       served: 588 -> 181.
 //   resid_sums (grid NC x B): every block re-derives its sequence's accepted length from the drafted
 //       tokens' ratios P_i(d_i) / q_i(d_i), then sums the correction weights max(0, P_a - q_a) (P_K
 //       when every draft is accepted) and P_a over its chunk of the vocabulary, in fp64.
@@ -29,7 +36,13 @@ namespace {
 constexpr int kT = 512;  // threads of the truncation block
 constexpr int kTW = kT / kWave;
 constexpr int kSample = 2048;
-constexpr int kCap = 8192;  // LDS collection capacity (values)
+constexpr int kCap = 12288;  // LDS collection capacity (values)
+constexpr int kSortCap = 8192;  // values sorted at a time (a power of two, <= kCap)
+constexpr int kTopCount = 1024;  // entries at the top of a row that are always collected
+constexpr int kU = 4;            // 16-byte loads in flight per thread
+constexpr int kTileV = kT * kU;  // vectors per tile of the streaming pass
+constexpr int kQueue = 320;      // a wave's queue: up to 63 waiting elements and 4 new ones per lane
+constexpr int kSub = 1024;       // sub-bins of the boundary bin
 constexpr int kBins = 256;  // digits of one radix pass
 constexpr int kMaxTopK = 4096;
 constexpr uint32_t kKeyLo = 0x00800000u;  // smallest finite key (key(-inf) + 1)
@@ -67,42 +80,77 @@ __device__ __forceinline__ int next_pow2(int n) {
   return p;
 }
 
+// Value histogram of the streaming pass: 2048 bins of 1/32 nat over d = y - mref in (-24, 40]
+// (mref = the sample max); bin 0 holds the largest values. Bin kNB is the spare bin: entries with d > 40, which are
+// caught afterwards from the row max and send the row to the radix select, and a few at the lower end. The
+// others with d <= -24, -inf entries, the banned id and padding lanes only add their mass to the total.
+// Each bin is one 64-bit LDS word: the count in bits 46..63 and, below, the sum of r * 2^26 with
+// r = exp(d - top of the bin) in (e^-1/32, 1]: one integer LDS atomic per element (fp64 and fp32 LDS
+// atomics measured several times slower on gfx950). Rows need V < 2^18 for the count field.
+constexpr int kNB = 2048;
+constexpr float kTop = 40.f;
+constexpr float kPerNat = 32.f;
+constexpr double kBinRatio = 0x1.f03f56a88b5d8p-1;  // exp(-1 / kPerNat): the scale of bin b + 1 over bin b
+constexpr int kSeg = 4;  // the streaming pass re-places its collection window between segments
+constexpr int kCountShift = 46;
+constexpr unsigned long long kMassMask = (1ull << kCountShift) - 1ull;
+constexpr int kMaxPackedV = (1 << 18) - 1;
+
+struct Shared {
+  float coll[kCap];
+  float queue[kTW][kQueue];  // each wave's elements above the floor, waiting for 64 to fold at once
+  unsigned long long hist[kNB + 1];
+  unsigned cnt[kBins];  // radix-select digits
+  double mass[kBins];
+  double red[kTW];
+  int n;
+  int ipar[6];
+  int wlo[kSeg], whi[kSeg];  // the window each segment collected (bins, inclusive)
+  int top[kSeg];             // and the bins [0, top)
+  int nseg[kSeg];            // collection fill after each segment
+  double dpar[4];
+  unsigned umax;
+};
+// The truncation block's LDS. Everything the kernel calls is inlined: with real functions for its rare steps it
+// needs a stack, and every launch was 10 us longer.
+__shared__ Shared sh;
+
 // ---------------------------------------------------------------- block reductions (512 threads)
-__device__ __forceinline__ double block_sum(double v, double* sh) {
+__device__ __forceinline__ double block_sum(double v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
   __syncthreads();
-  if (threadIdx.x % kWave == 0) sh[threadIdx.x / kWave] = v;
+  if (threadIdx.x % kWave == 0) sh.red[threadIdx.x / kWave] = v;
   __syncthreads();
   double t = 0.0;
 #pragma unroll
-  for (int w = 0; w < kTW; ++w) t += sh[w];
+  for (int w = 0; w < kTW; ++w) t += sh.red[w];
   return t;
 }
-__device__ __forceinline__ float block_max(float v, double* sh) {
+__device__ __forceinline__ float block_max(float v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, kWave));
   __syncthreads();
-  if (threadIdx.x % kWave == 0) sh[threadIdx.x / kWave] = v;
+  if (threadIdx.x % kWave == 0) sh.red[threadIdx.x / kWave] = v;
   __syncthreads();
   float t = -INFINITY;
 #pragma unroll
-  for (int w = 0; w < kTW; ++w) t = fmaxf(t, (float)sh[w]);
+  for (int w = 0; w < kTW; ++w) t = fmaxf(t, (float)sh.red[w]);
   return t;
 }
-__device__ __forceinline__ int block_isum(int v, double* sh) {
+__device__ __forceinline__ int block_isum(int v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
   __syncthreads();
-  if (threadIdx.x % kWave == 0) sh[threadIdx.x / kWave] = (double)v;
+  if (threadIdx.x % kWave == 0) sh.red[threadIdx.x / kWave] = (double)v;
   __syncthreads();
   int t = 0;
 #pragma unroll
-  for (int w = 0; w < kTW; ++w) t += (int)sh[w];
+  for (int w = 0; w < kTW; ++w) t += (int)sh.red[w];
   return t;
 }
 // Exclusive prefix sum over the block in thread order; *total gets the block total.
-__device__ __forceinline__ double block_excl_scan(double v, double* sh, double* total) {
+__device__ __forceinline__ double block_excl_scan(double v, double* total) {
   const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
   double inc = v;
 #pragma unroll
@@ -113,21 +161,41 @@ __device__ __forceinline__ double block_excl_scan(double v, double* sh, double* 
   double ex = __shfl_up(inc, 1, kWave);
   if (lane == 0) ex = 0.0;
   __syncthreads();
-  if (lane == kWave - 1) sh[w] = inc;
+  if (lane == kWave - 1) sh.red[w] = inc;
   __syncthreads();
   double base = 0.0, tot = 0.0;
 #pragma unroll
   for (int i = 0; i < kTW; ++i) {
-    base += (i < w) ? sh[i] : 0.0;
-    tot += sh[i];
+    base += (i < w) ? sh.red[i] : 0.0;
+    tot += sh.red[i];
   }
   *total = tot;
   return base + ex;
 }
 
 // Bitonic sort, descending, of s[0..n) (n a power of two); starts and ends with a barrier.
-__device__ void sort_desc(float* s, int n) {
+__device__ void sort_desc(int n) {
+  float* s = sh.coll;
   __syncthreads();
+  if (n <= kT) {  // a few elements per lane of one wave, whose LDS operations complete in order: no barriers
+    if (threadIdx.x < kWave) {
+      for (int k = 2; k <= n; k <<= 1)
+        for (int j = k >> 1; j > 0; j >>= 1) {
+          for (int i = threadIdx.x; i < (n >> 1); i += kWave) {
+            const int lo = ((i & ~(j - 1)) << 1) | (i & (j - 1));
+            const int hi = lo + j;
+            const float a = s[lo], b = s[hi];
+            const bool sw = (lo & k) == 0 ? a < b : a > b;
+            s[lo] = sw ? b : a;
+            s[hi] = sw ? a : b;
+          }
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+        }
+    }
+    __syncthreads();
+    return;
+  }
   for (int k = 2; k <= n; k <<= 1)
     for (int j = k >> 1; j > 0; j >>= 1) {
       for (int i = threadIdx.x; i < (n >> 1); i += kT) {
@@ -146,49 +214,56 @@ __device__ void sort_desc(float* s, int n) {
 
 // Appends y (where pred) to s_coll through one LDS counter bump per wave; the counter keeps counting
 // past kCap so that an overflow is visible. Called by every lane of the wave.
-__device__ __forceinline__ void append(float y, bool pred, float* s_coll, int* s_n) {
+__device__ __forceinline__ void append(float y, bool pred) {
   const uint64_t bal = __ballot(pred);
   if (bal == 0) return;
   const int lane = threadIdx.x % kWave;
   int base = 0;
-  if (lane == 0) base = atomicAdd(s_n, __popcll(bal));
+  if (lane == 0) base = atomicAdd(&sh.n, __popcll(bal));
   base = __shfl(base, 0, kWave);
   const int slot = base + __popcll(bal & ((1ull << lane) - 1ull));
-  if (pred && slot < kCap) s_coll[slot] = y;
+  if (pred && slot < kCap) sh.coll[slot] = y;
 }
 
+// A row as its 16-byte aligned vectors [0, n4) and the <= 6 elements in front of and behind them (a row
+// of an odd vocabulary starts anywhere in a 16-byte line).
+struct RowView {
+  const float* row;
+  const u32x4* body;
+  int pre, n4, V;
+  __device__ RowView(const float* r, int v) : row(r), V(v) {
+    pre = min((int)((0u - (unsigned)((uintptr_t)r >> 2)) & 3u), v);
+    body = reinterpret_cast<const u32x4*>(r + pre);
+    n4 = (v - pre) >> 2;
+  }
+  // id of edge element j (the elements outside the vectors, in order), V past the last one
+  __device__ int edge(int j) const { return min(j < pre ? j : j + 4 * n4, V); }
+};
+
 // Calls f(y, ix, valid) for every element of a row; U 16-byte loads in flight per thread.
-template <bool kDiv, bool kVec, int U = 4, typename F>
-__device__ __forceinline__ void for_each_y(const float* row, int V, double rt, int ban, F&& f) {
+template <bool kDiv, int U = 4, typename F>
+__device__ __forceinline__ void for_each_y(const RowView& rv, double rt, int ban, F&& f) {
   const int tid = threadIdx.x;
-  int done = 0;
-  if (kVec) {
-    const u32x4* row4 = reinterpret_cast<const u32x4*>(row);
-    const int n4 = V >> 2;
-    for (int base = 0; base < n4; base += kT * U) {
-      u32x4 x[U];
+  for (int base = 0; base < rv.n4; base += kT * U) {
+    u32x4 x[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const u32x4* p = row4 + min(base + u * kT + tid, n4 - 1);
-        x[u] = *p;
-      }
+    for (int u = 0; u < U; ++u) x[u] = rv.body[min(base + u * kT + tid, rv.n4 - 1)];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int j = base + u * kT + tid;
-        const bool ok = j < n4;
-        const float xs[4] = {__uint_as_float(x[u].x), __uint_as_float(x[u].y), __uint_as_float(x[u].z),
-                             __uint_as_float(x[u].w)};
+    for (int u = 0; u < U; ++u) {
+      const int j = base + u * kT + tid;
+      const bool ok = j < rv.n4;
+      const float xs[4] = {__uint_as_float(x[u].x), __uint_as_float(x[u].y), __uint_as_float(x[u].z),
+                           __uint_as_float(x[u].w)};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) f(make_y<kDiv>(xs[e], 4 * j + e, rt, ban), 4 * j + e, ok);
+      for (int e = 0; e < 4; ++e) {
+        const int ix = rv.pre + 4 * j + e;
+        f(make_y<kDiv>(xs[e], ix, rt, ban), ix, ok);
       }
     }
-    done = n4 << 2;
   }
-  for (int base = done; base < V; base += kT) {
-    const int ix = base + tid;
-    const bool ok = ix < V;
-    f(make_y<kDiv>(row[ok ? ix : V - 1], ix, rt, ban), ix, ok);
-  }
+  const int ix = rv.edge(tid);
+  const bool ok = ix < rv.V;
+  f(make_y<kDiv>(rv.row[ok ? ix : 0], ix, rt, ban), ix, ok);
 }
 
 struct TruncArgs {
@@ -209,31 +284,11 @@ struct TruncArgs {
   int* passes_out;
 };
 
-// Value histogram of the streaming pass: 2048 bins of 1/32 nat over d = y - mref in (-24, 40]
-// (mref = the sample max); bin 0 holds the largest values. Bin kNB is the spare bin: entries with
-// d <= -24, -inf entries, the banned id and padding lanes land there (its mass still counts towards
-// the total). d > 40 is caught afterwards from the row max and sends the row to the radix select.
-// Each bin is one 64-bit LDS word: the count in bits 46..63 and, below, the sum of r * 2^26 with
-// r = exp(d - top of the bin) in (e^-1/32, 1]: one integer LDS atomic per element (fp64 and fp32 LDS
-// atomics measured several times slower on gfx950). Rows need V < 2^18 for the count field.
-constexpr int kNB = 2048;
-constexpr float kTop = 40.f;
-constexpr float kPerNat = 32.f;
-constexpr double kBinRatio = 0x1.f03f56a88b5d8p-1;  // exp(-1 / kPerNat): the scale of bin b + 1 over bin b
-constexpr int kSeg = 4;  // the streaming pass re-places its collection window between segments
-constexpr int kCountShift = 46;
-constexpr unsigned long long kMassMask = (1ull << kCountShift) - 1ull;
-constexpr int kMaxPackedV = (1 << 18) - 1;
-
 // Bin of an element from its raw logit x: t = 32 (40 - d) with d = x / T - mref, as one fma whose
 // coefficients the block derives once (tA = -32 / T, tB = 32 (40 + mref)). Monotone in x.
 __device__ __forceinline__ unsigned bin_of_t(float t) {
   return min((unsigned)(int)__builtin_amdgcn_fmed3f(t, -1.f, (float)kNB), (unsigned)kNB);
 }
-// c ? x : y on values: a conditional over two array elements (lvalues) selects their addresses, which
-// sends register arrays to scratch memory
-__device__ __forceinline__ double pick(bool c, double x, double y) { return c ? x : y; }
-
 // exp(top of the bin) relative to exp(mref); consecutive bins scale by kBinRatio
 __device__ __forceinline__ double bin_scale(int bin) { return exp((double)kTop - (double)bin / kPerNat); }
 __device__ __forceinline__ double bin_mass(unsigned long long h, double scale) {  // relative to exp(mref)
@@ -241,69 +296,77 @@ __device__ __forceinline__ double bin_mass(unsigned long long h, double scale) {
 }
 
 struct BinMap {  // the per-row coefficients of the element -> bin / exponent maps
-  float tA, tB;  // t = fma(x, tA, tB)
-  float rf, nm;  // d = fma(x, rf, nm) = x / T - mref
+  float tA, tB;       // t = fma(x, tA, tB)
+  float rf, rl, nm;   // d = x (rf + rl) + nm = x / T - mref
+  float eA, eB;       // exp(d) = exp2(fma(x, eA, eB)) * cold_scale
+  double cold_scale;  // what the rounding of eB took away
   __device__ unsigned bin(float x) const { return bin_of_t(fmaf(x, tA, tB)); }
-};
-
-struct Shared {
-  float coll[kCap];
-  unsigned long long hist[kNB + 1];
-  unsigned cnt[kBins];  // radix-select digits
-  double mass[kBins];
-  double red[kTW];
-  int n;
-  int ipar[4];
-  int wlo[kSeg], whi[kSeg];  // the window each segment collected (bins, inclusive)
-  int nseg[kSeg];            // collection fill after each segment
-  double dpar[4];
-  unsigned umax;
+  // an element's histogram entry: a count of one and its mass relative to its bin's upper edge
+  __device__ unsigned long long packed(float x, unsigned bin) const {
+    const float d = fmaf(x, rl, fmaf(x, rf, nm));
+    const float edge = fmaf((float)bin, -1.f / kPerNat, kTop);
+    const float r = __builtin_amdgcn_exp2f((d - edge) * 1.44269504f) * 0x1p26f;
+    return (1ull << kCountShift) | (unsigned long long)(unsigned)r;
+  }
+  __device__ void set(double rt, float mref) {
+    rf = (float)rt;
+    rl = (float)(rt - (double)rf);
+    tA = -kPerNat * rf;
+    tB = kPerNat * (kTop + mref);
+    nm = -mref;
+    const double l2e = 1.4426950408889634;
+    eA = (float)(rt * l2e);
+    eB = (float)(-(double)mref * l2e);
+    cold_scale = exp2(-(double)mref * l2e - (double)eB);
+  }
 };
 
 // Count of j < lim with base + sum_{i<j} e_i < target, e_i = exp(s_i - m) in fp64 (a prefix, since
 // the partial sums only grow); *tot = sum_{j<lim} e_j.
-__device__ int count_below(const float* s, int lim, double m, double base, double target, double* tot,
-                           double* sh) {
+__device__ int count_below(int lim, double m, double base, double target, double* tot) {
+  const float* s = sh.coll;
   const int L = (lim + kT - 1) / kT;
   const int j0 = min(lim, (int)threadIdx.x * L), j1 = min(lim, j0 + L);
   double loc = 0.0;
   for (int j = j0; j < j1; ++j) loc += exp((double)s[j] - m);
-  const double ex = block_excl_scan(loc, sh, tot);
+  const double ex = block_excl_scan(loc, tot);
   int c = 0;
   double run = base + ex;
   for (int j = j0; j < j1; ++j) {
     c += run < target;
     run += exp((double)s[j] - m);
   }
-  return block_isum(c, sh);
+  return block_isum(c);
 }
 
 // sum over j < n with s_j >= thr of exp(s_j - m)
-__device__ __forceinline__ double mass_at_least(const float* s, int n, float thr, double m, double* sh) {
+__device__ double mass_at_least(int n, float thr, double m) {
+  const float* s = sh.coll;
   double loc = 0.0;
   for (int j = threadIdx.x; j < n; j += kT) loc += (s[j] >= thr) ? exp((double)s[j] - m) : 0.0;
-  return block_sum(loc, sh);
+  return block_sum(loc);
 }
 
-__device__ int count_cmp(const float* s, int n, float v, bool strictly_greater, double* sh) {
+__device__ int count_cmp(int n, float v, bool strictly_greater) {
+  const float* s = sh.coll;
   int c = 0;
   for (int j = threadIdx.x; j < n; j += kT) c += strictly_greater ? (s[j] > v) : (s[j] == v);
-  return block_isum(c, sh);
+  return block_isum(c);
 }
 
 // Pads the collection to a power of two with -inf and sorts it (descending).
-__device__ void sort_collection(Shared& sh, int n) {
+__device__ void sort_collection(int n) {
   const int np = next_pow2(max(n, 2));
   for (int j = n + threadIdx.x; j < np; j += kT) sh.coll[j] = -INFINITY;
-  sort_desc(sh.coll, np);
+  sort_desc(np);
 }
 
 // One fallback pass over the keys: counts/mass (relative to the exact max m) above khi, and either a
 // histogram of [klo, khi] in digits of 2^shift keys or a collection of that range. On want_z it also
 // sums the whole row's mass and counts its finite entries.
-template <bool kDiv, bool kVec, bool kHist>
-__device__ void range_pass(const float* row, const TruncArgs& a, float m, uint32_t klo, uint32_t khi, int shift,
-                           bool want_z, Shared& sh, int* ca_out, double* ma_out, double* z_out, int* cf_out) {
+template <bool kDiv, bool kHist>
+__device__ void range_pass(const RowView& rv, const TruncArgs& a, float m, uint32_t klo, uint32_t khi, int shift,
+                           bool want_z, int* ca_out, double* ma_out, double* z_out, int* cf_out) {
   if (kHist)
     for (int j = threadIdx.x; j < kBins; j += kT) {
       sh.cnt[j] = 0u;
@@ -313,7 +376,7 @@ __device__ void range_pass(const float* row, const TruncArgs& a, float m, uint32
   __syncthreads();
   int ca = 0, cf = 0;
   double ma = 0.0, z = 0.0;
-  for_each_y<kDiv, kVec, 2>(row, a.V, a.rt, a.ban, [&](float y, int ix, bool ok) {
+  for_each_y<kDiv, 2>(rv, a.rt, a.ban, [&](float y, int ix, bool ok) {
     const bool fin = ok && (y > -INFINITY);
     const uint32_t key = fkey(y);
     const float e = __expf(y - m);
@@ -332,22 +395,22 @@ __device__ void range_pass(const float* row, const TruncArgs& a, float m, uint32
         atomicAdd(&sh.mass[bin], (double)e);
       }
     } else {
-      append(y, in, sh.coll, &sh.n);
+      append(y, in);
     }
   });
-  *ca_out = block_isum(ca, sh.red);
-  *ma_out = block_sum(ma, sh.red);
+  *ca_out = block_isum(ca);
+  *ma_out = block_sum(ma);
   if (want_z) {
-    *z_out = block_sum(z, sh.red);
-    *cf_out = block_isum(cf, sh.red);
+    *z_out = block_sum(z);
+    *cf_out = block_isum(cf);
   }
   __syncthreads();
 }
 
 // Exact radix select with the exact row max m. Count mode (use_k): the top_k-th largest value; mass
 // mode: the smallest y whose strictly-greater mass is < top_p * Z. Writes thr / Zk (relative to m).
-template <bool kDiv, bool kVec>
-__device__ void radix_resolve(const float* row, const TruncArgs& a, float m, bool use_k, bool use_p, Shared& sh,
+template <bool kDiv>
+__device__ __forceinline__ void radix_resolve(const RowView& rv, const TruncArgs& a, float m, bool use_k, bool use_p,
                               float* thr_out, double* zk_out, int* passes) {
   const double md = (double)m;
   uint32_t klo = kKeyLo, khi = kKeyHi;
@@ -363,7 +426,7 @@ __device__ void radix_resolve(const float* row, const TruncArgs& a, float m, boo
   double zk = 0.0;
   bool resolved = false;
   for (int it = 0; !resolved; ++it) {
-    range_pass<kDiv, kVec, true>(row, a, m, klo, khi, shift, it == 0, sh, &ca, &ma, &z, &cf);
+    range_pass<kDiv, true>(rv, a, m, klo, khi, shift, it == 0, &ca, &ma, &z, &cf);
     ++*passes;
     if (it == 0) {
       Z = z;
@@ -415,25 +478,25 @@ __device__ void radix_resolve(const float* row, const TruncArgs& a, float m, boo
         zk = cum + bmass;
       }
       resolved = true;
-    } else if (cnt <= (unsigned)kCap) {
+    } else if (cnt <= (unsigned)kSortCap) {
       klo = nlo;
       khi = nhi;
       int ca2 = 0, cf2 = 0;
       double ma2 = 0.0, z2 = 0.0;
-      range_pass<kDiv, kVec, false>(row, a, m, klo, khi, 0, false, sh, &ca2, &ma2, &z2, &cf2);
+      range_pass<kDiv, false>(rv, a, m, klo, khi, 0, false, &ca2, &ma2, &z2, &cf2);
       ++*passes;
-      const int n = min(sh.n, kCap);
-      sort_collection(sh, n);
+      const int n = min(sh.n, kSortCap);
+      sort_collection(n);
       if (count_mode) {
         v = sh.coll[min(max(k - 1 - ca2, 0), max(n - 1, 0))];
-        c_gt = ca2 + count_cmp(sh.coll, n, v, true, sh.red);
-        c_eq = count_cmp(sh.coll, n, v, false, sh.red);
+        c_gt = ca2 + count_cmp(n, v, true);
+        c_eq = count_cmp(n, v, false);
       } else {
         double tot = 0.0;
-        int nk = count_below(sh.coll, n, md, ma2, tp, &tot, sh.red);
+        int nk = count_below(n, md, ma2, tp, &tot);
         nk = min(max(nk, 1), n);
         v = sh.coll[nk - 1];
-        zk = ma2 + mass_at_least(sh.coll, n, v, md, sh.red);
+        zk = ma2 + mass_at_least(n, v, md);
       }
       resolved = true;
     } else {
@@ -453,33 +516,33 @@ __device__ void radix_resolve(const float* row, const TruncArgs& a, float m, boo
   int ca2 = 0, cf2 = 0;
   double ma2 = 0.0, z2 = 0.0;
   const uint32_t kk = fkey(kth);
-  range_pass<kDiv, kVec, false>(row, a, m, kk + 1u, kKeyHi, 0, false, sh, &ca2, &ma2, &z2, &cf2);
+  range_pass<kDiv, false>(rv, a, m, kk + 1u, kKeyHi, 0, false, &ca2, &ma2, &z2, &cf2);
   ++*passes;
-  const int n = min(sh.n, kCap);
-  sort_collection(sh, n);
+  const int n = min(sh.n, kSortCap);
+  sort_collection(n);
   const double e_k = exp((double)kth - md);
   double s_gt = 0.0;
   const double copies = (double)(k - c_gt);
   if (use_p) {
     double tot = 0.0;
     // total first: S = sum_{coll} e + copies * e_k
-    (void)count_below(sh.coll, n, md, 0.0, -1.0, &tot, sh.red);
+    (void)count_below(n, md, 0.0, -1.0, &tot);
     s_gt = tot;
     const double target = (double)a.top_p * (s_gt + copies * e_k);
-    int nk = count_below(sh.coll, n, md, 0.0, target, &tot, sh.red);
+    int nk = count_below(n, md, 0.0, target, &tot);
     int ncp = 0;
     for (int i = threadIdx.x; i < k - c_gt; i += kT) ncp += (s_gt + (double)i * e_k) < target;
-    ncp = block_isum(ncp, sh.red);
+    ncp = block_isum(ncp);
     nk = max(nk + ncp, 1);
     if (nk <= c_gt) {
       const float thr = sh.coll[nk - 1];
       *thr_out = thr;
-      *zk_out = mass_at_least(sh.coll, n, thr, md, sh.red);
+      *zk_out = mass_at_least(n, thr, md);
       return;
     }
   } else {
     double tot = 0.0;
-    (void)count_below(sh.coll, n, md, 0.0, -1.0, &tot, sh.red);
+    (void)count_below(n, md, 0.0, -1.0, &tot);
     s_gt = tot;
   }
   *thr_out = kth;
@@ -489,262 +552,482 @@ __device__ void radix_resolve(const float* row, const TruncArgs& a, float m, boo
 // Keeps the collected logits whose bin lies in [lo, hi] and that came from a segment in the bit set
 // `segs` (entry j came from segment s when nseg[s-1] <= j < nseg[s]), packed at the front of
 // sh.coll; returns how many.
-__device__ __forceinline__ int compact_bins(Shared& sh, const BinMap& bm, int n, int lo, int hi, unsigned segs) {
+__device__ __forceinline__ int compact_bins(const BinMap& bm, int n, int lo, int hi, unsigned segs) {
   constexpr int kPer = kCap / kT;
   float v[kPer];
-  bool kp[kPer];
-  int keep = 0;
+  unsigned kp = 0u;
+  const bool all = segs == (1u << kSeg) - 1u;
 #pragma unroll
   for (int u = 0; u < kPer; ++u) {
-    const int j = (int)threadIdx.x * kPer + u;
+    if (u * kT >= n) break;  // block-uniform
+    const int j = u * kT + (int)threadIdx.x;
     v[u] = j < n ? sh.coll[j] : -INFINITY;
     const int bin = (int)bm.bin(v[u]);
-    int s = 0;
-    while (s < kSeg - 1 && j >= sh.nseg[s]) ++s;
-    kp[u] = (j < n) && bin >= lo && bin <= hi && ((segs >> s) & 1u);
-    keep += kp[u];
+    bool keep = j < n && bin >= lo && bin <= hi;
+    if (!all) {
+      int s = 0;
+      while (s < kSeg - 1 && j >= sh.nseg[s]) ++s;
+      keep = keep && ((segs >> s) & 1u);
+    }
+    kp |= (unsigned)keep << u;
   }
   double tot = 0.0;
-  int w = (int)block_excl_scan((double)keep, sh.red, &tot);  // every read of sh.coll precedes its barriers
+  int w = (int)block_excl_scan((double)__popc(kp), &tot);  // every read of sh.coll precedes its barriers
 #pragma unroll
   for (int u = 0; u < kPer; ++u)
-    if (kp[u]) sh.coll[w++] = v[u];
+    if ((kp >> u) & 1u) sh.coll[w++] = v[u];
   __syncthreads();
   return (int)tot;
 }
 
-// Appends the values of xv whose bit is set in mask. Called by every lane of the wave: the lanes'
-// offsets are the wave-exclusive prefix of their counts, summed from the counts' bit planes (a ballot
-// and a masked bit count each), and one LDS counter bump per wave takes the wave's total (same-address
-// LDS atomics serialise, one lane after another).
-template <int N>
-__device__ __forceinline__ void append_batch(const float (&xv)[N], unsigned mask, Shared& sh) {
-  constexpr int kPlanes = N >= 16 ? 5 : N >= 8 ? 4 : N >= 4 ? 3 : N >= 2 ? 2 : 1;  // bits of a count <= N
-  const int c = __popc(mask);
-  int pre = 0, tot = 0;
-#pragma unroll
-  for (int bit = 0; bit < kPlanes; ++bit) {
-    const uint64_t bb = __ballot((c >> bit) & 1);
-    pre += (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bb, 0u)) << bit;
-    tot += __popcll(bb) << bit;
-  }
-  if (tot == 0) return;  // wave-uniform
-  int base = 0;
-  if (threadIdx.x % kWave == 0) base = atomicAdd(&sh.n, tot);
-  int pos = __builtin_amdgcn_readfirstlane(base) + pre;
-#pragma unroll
-  for (int e = 0; e < N; ++e)
-    if ((mask >> e) & 1u) {
-      if (pos < kCap) sh.coll[pos] = xv[e];
-      ++pos;
-    }
+// Segment s of the streaming pass: the row's tiles (kTileV vectors, the last one partial) number 0 mod 16;
+// the other multiples of 4; the other even ones; the odd ones: 1/16, 3/16, 1/4 and 1/2 of the row, each
+// spread over all of it (token ids are not exchangeable: a vocabulary's first ids are its frequent tokens).
+// The edge elements belong to segment 0.
+__device__ __forceinline__ int seg_tile(int s, int i) {
+  if (s == 0) return 16 * i;
+  if (s == 1) return 16 * (i / 3) + 4 * (i % 3 + 1);
+  return s == 2 ? 4 * i + 2 : 2 * i + 1;
+}
+__device__ __forceinline__ int seg_size(const RowView& rv, int s) {
+  const int nt = (rv.n4 + kTileV - 1) / kTileV, n16 = (nt + 15) / 16;
+  const int cnt = s == 0 ? n16 : s == 1 ? (nt + 3) / 4 - n16 : s == 2 ? (nt + 1) / 4 : nt / 2;
+  const int tl = nt - 1, sl = (tl & 1) ? 3 : (tl & 2) ? 2 : (tl & 15) ? 1 : 0;  // the last tile's segment
+  int n = 4 * cnt * kTileV;
+  if (nt > 0 && s == sl) n -= 4 * (nt * kTileV - rv.n4);
+  return s == 0 ? n + rv.V - 4 * rv.n4 : n;
 }
 
-// Streams the row's elements [e0, e1) (e0 and e1 multiples of 4 on the vector path, except e1 = V),
-// in the logits' own units: the division by the temperature is folded into the bin / exponent maps,
-// and the exact y = x / T is only formed for the few collected values.
-// kHist: histogram every element, track the max and the NaN flag, collect the bins [wlo, whi].
-// Otherwise only collect the bins [wlo, whi]. The element body is branch-free; the banned id and the
-// padding lanes of a last partial tile take a separate path for that tile only.
-template <bool kVec, bool kHist>
-__device__ void stream_segment(const float* row, const TruncArgs& a, const BinMap& bm, int e0, int e1, int wlo,
-                               int whi, Shared& sh, float& mx, unsigned& nanbits) {
-  constexpr int U = 4;
-  const int tid = threadIdx.x;
+// The logit below which no element has a bin < b: bin b's lower edge, half a bin and the rounding of the
+// element -> bin map further down.
+__device__ __forceinline__ float below_bin(const BinMap& bm, int b) {
+  return (bm.tB - ((float)b + 0.5f + 1e-6f * fabsf(bm.tB))) / -bm.tA;
+}
+
+// Streams a segment of the row in the logits' own units: the division by the temperature is folded into
+// the bin / exponent maps, and the exact y = x / T is only formed for the few collected values.
+// kHist: elements above x_lo (which lies below the floor, below_bin) wait in their wave's queue; each full
+// wave of 64 goes to the histogram and, those with a bin in [wlo, whi] or below `top`, to the collection.
+// The others only add their mass (relative to exp(mref), less the rounding of bm.eB) to `tail`: fp32 over a
+// tile's 16 elements of a thread, fp64 across tiles. Without the queue every wave would run the 30 instructions of the
+// histogram for each of its elements, as some lane always has one above the floor (the block issues 16 waves'
+// instructions per CU, and the pass was bound by that: 33 a element, now 15 and 35 per element above the
+// floor); and below the histogram's range its LDS atomics all met in one bin. A NaN makes `tail` NaN.
+// Otherwise only the elements between x_lo and x_hi are looked at, and those of the bins [wlo, whi] collected.
+template <bool kHist>
+__device__ __forceinline__ void stream_segment(const RowView& rv, const TruncArgs& a, const BinMap& bm, int s, float x_lo,
+                                               float x_hi, int top, int wlo, int whi, float& mx, double& tail) {
+  const int tid = threadIdx.x, lane = tid % kWave;
+  float* queue = sh.queue[tid / kWave];
+  int fill = 0;  // wave-uniform
   const unsigned wspan = (unsigned)(whi - wlo);
-  auto one = [&](float x, unsigned& mask, int e) {
-    const unsigned bin = bm.bin(x);
-    if (kHist) {
-      const float d = fmaf(x, bm.rf, bm.nm);
-      const float top = fmaf((float)bin, -1.f / kPerNat, kTop);
-      const float r = __builtin_amdgcn_exp2f(fmaf(d - top, 1.44269504f, 26.f));  // r * 2^26
-      atomicAdd(&sh.hist[bin], (1ull << kCountShift) | (unsigned long long)(unsigned)r);
-      mx = fmaxf(mx, x);
-      nanbits = max(nanbits, __float_as_uint(x) << 1);  // a NaN sorts above +-inf here
+  // folds the n (<= 64) elements at the end of the queue
+  auto fold = [&](int n) {
+    fill -= n;
+    bool in = false;
+    float x = 0.f;
+    if (lane < n) {
+      x = queue[fill + lane];
+      const unsigned bin = bm.bin(x);
+      if (kHist) {
+        atomicAdd(&sh.hist[bin], bm.packed(x, bin));
+        in = (int)bin < top;
+      }
+      in |= (unsigned)((int)bin - wlo) <= wspan;
     }
-    mask |= (unsigned)((unsigned)((int)bin - wlo) <= wspan) << e;
+    append(x, in);
   };
-  int t0 = e0;
-  if (kVec) {
-    const u32x4* row4 = reinterpret_cast<const u32x4*>(row);
-    const int v0 = e0 >> 2, v1 = (e1 == a.V) ? (a.V >> 2) : (e1 >> 2);
-    const int vb = a.ban >= 0 ? (a.ban >> 2) : -1;
-    // the next tile's loads are issued before the current tile is folded, so the fold hides their
-    // latency; addresses are clamped to the last vector (the last tile's prefetch reads one line)
-    auto load = [&](u32x4 (&dst)[U], int base) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) dst[u] = row4[min(base + u * kT + tid, v1 - 1)];
-    };
-    u32x4 xn[U];
-    if (v0 < v1) load(xn, v0);
-    for (int base = v0; base < v1; base += kT * U) {
-      u32x4 x[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) x[u] = xn[u];
-      load(xn, base + kT * U);
-      float xv[4 * U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        xv[4 * u + 0] = __uint_as_float(x[u].x);
-        xv[4 * u + 1] = __uint_as_float(x[u].y);
-        xv[4 * u + 2] = __uint_as_float(x[u].z);
-        xv[4 * u + 3] = __uint_as_float(x[u].w);
-      }
-      // wave-uniform: does this tile hold the banned id or padding lanes?
-      if (base + kT * U > v1 || (unsigned)(vb - base) < (unsigned)(kT * U)) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const int j = base + u * kT + tid;
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (j >= v1 || 4 * j + e == a.ban) xv[4 * u + e] = -INFINITY;
-        }
-      }
-      unsigned mask = 0u;
-#pragma unroll
-      for (int e = 0; e < 4 * U; ++e) one(xv[e], mask, e);
-      append_batch(xv, mask, sh);
+  auto push = [&](float x, bool hot) {
+    const uint64_t bal = __ballot(hot);
+    if (bal == 0) return;
+    if (hot)
+      queue[fill + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u))] = x;
+    fill += __popcll(bal);
+  };
+  auto one = [&](float x, float& cold) {
+    bool hot = x > x_lo;
+    if (kHist) {
+      mx = fmaxf(mx, x);
+      const float e = __builtin_amdgcn_exp2f(fmaf(x, bm.eA, bm.eB));
+      cold += hot ? 0.f : e;
+    } else {
+      hot = hot && x < x_hi;
     }
-    t0 = max(e0, v1 << 2);
+    push(x, hot);
+  };
+  // the next tile's loads are issued before the current tile is folded, so the fold hides their
+  // latency; addresses are clamped to the last vector
+  const int n4 = rv.n4;
+  auto load = [&](u32x4 (&dst)[kU], int tile) {
+#pragma unroll
+    for (int u = 0; u < kU; ++u) dst[u] = rv.body[min(tile * kTileV + u * kT + tid, n4 - 1)];
+  };
+  const int nt = (n4 + kTileV - 1) / kTileV;
+  u32x4 xn[kU];
+  int tile = seg_tile(s, 0);
+  if (tile < nt) load(xn, tile);
+  for (int i = 0; tile < nt; ++i) {
+    const int base = tile * kTileV;
+    u32x4 x[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) x[u] = xn[u];
+    tile = seg_tile(s, i + 1);
+    if (tile < nt) load(xn, tile);
+    // block-uniform: does this tile hold the banned id or padding lanes?
+    const int e0 = rv.pre + 4 * base;
+    const bool odd = base + kTileV > n4 || (unsigned)(a.ban - e0) < (unsigned)(4 * kTileV);
+    float cold = 0.f;
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      float xv[4] = {__uint_as_float(x[u].x), __uint_as_float(x[u].y), __uint_as_float(x[u].z), __uint_as_float(x[u].w)};
+      if (odd) {
+        const int j = base + u * kT + tid;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (j >= n4 || rv.pre + 4 * j + e == a.ban) xv[e] = -INFINITY;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) one(xv[e], cold);
+      while (fill >= kWave) fold(kWave);
+    }
+    if (kHist) tail += (double)cold;
   }
-  for (int base = t0; base < e1; base += kT) {
-    const int ix = base + tid;
-    float xv[1];
-    xv[0] = (ix < e1 && ix != a.ban) ? row[ix < e1 ? ix : e1 - 1] : -INFINITY;
-    unsigned mask = 0u;
-    one(xv[0], mask, 0);
-    append_batch(xv, mask, sh);
+  if (s == 0 && tid < kWave) {
+    const int ix = rv.edge(tid);
+    float cold = 0.f;
+    one(ix < rv.V && ix != a.ban ? rv.row[ix] : -INFINITY, cold);
+    if (kHist) tail += (double)cold;
   }
+  while (fill > 0) fold(min(fill, kWave));
 }
 
-// Element bounds of segment s of the streaming pass.
-template <bool kVec>
-__device__ __forceinline__ void seg_bounds(int V, int s, int* e0, int* e1) {
-  if (kVec) {
-    const int n4 = V >> 2;
-    *e0 = 4 * (int)((int64_t)n4 * s / kSeg);
-    *e1 = s == kSeg - 1 ? V : 4 * (int)((int64_t)n4 * (s + 1) / kSeg);
-  } else {
-    *e0 = (int)((int64_t)V * s / kSeg);
-    *e1 = (int)((int64_t)V * (s + 1) / kSeg);
+// ---------------------------------------------------------------- the histogram, read by one wave
+// The steps between the segments run on the block's first wave: across all eight, the same few values computed
+// by each, they cost the CU's two blocks 17k cycles apiece (7 us alone, 45 us beside a streaming block).
+// Lane l holds the 32 bins [32 l, 32 l + 32) of the histogram: their mass (relative to exp(mref)) and count, and
+// the inclusive sums over the lanes.
+constexpr int kLB = kNB / kWave;
+static_assert(kLB == 32, "a lane's bins are one nat");
+struct LaneBins {
+  double sc;        // bin_scale(32 l)
+  double rk;        // kBinRatio^(l % 32)
+  double im;        // inclusive mass
+  unsigned ic;      // inclusive count
+  double m;
+  unsigned c;
+  __device__ void init() {
+    const int lane = threadIdx.x % kWave;
+    sc = bin_scale(lane * kLB);
+    rk = exp(-(double)(lane % kLB) / (double)kPerNat);
   }
+  __device__ void load() {
+    const int lane = threadIdx.x % kWave, k0 = lane % kLB;
+    double ms = 0.0, r = sc * rk * 0x1p-26;
+    unsigned cs = 0u;
+    // bin (l + i) % 32 at step i: the lanes' reads fall on all banks
+#pragma unroll 4
+    for (int i = 0; i < kLB; ++i) {
+      const int k = (k0 + i) % kLB;
+      const unsigned long long h = sh.hist[lane * kLB + k];
+      cs += (unsigned)(h >> kCountShift);
+      ms += (double)(h & kMassMask) * r;
+      r *= k == kLB - 1 ? kBinRatio * 0x1.5bf0a8b145769p+1 : kBinRatio;  // wraps by a factor of e
+    }
+    m = ms;
+    c = cs;
+    im = ms;
+    ic = cs;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const double om = __shfl_up(im, off, kWave);
+      const unsigned oc = (unsigned)__shfl_up((int)ic, off, kWave);
+      im += lane >= off ? om : 0.0;
+      ic += lane >= off ? oc : 0u;
+    }
+  }
+  __device__ double mass() const { return __shfl(im, kWave - 1, kWave); }
+  // the first bin at which the cumulative mass reaches tgt (> 0), -1 if none does; *before: the mass above it
+  __device__ int find_mass(double tgt, double* before) const {
+    const int lane = threadIdx.x % kWave;
+    const uint64_t hit = __ballot(im >= tgt);
+    if (hit == 0) return -1;
+    const int L = __builtin_ctzll(hit);
+    const double base = L > 0 ? __shfl(im, L - 1, kWave) : 0.0;
+    const double sl = __shfl(sc, L, kWave) * rk * 0x1p-26;
+    const double add = lane < kLB ? (double)(sh.hist[L * kLB + lane % kLB] & kMassMask) * sl : 0.0;
+    double inc = add;
+#pragma unroll
+    for (int off = 1; off < kLB; off <<= 1) {
+      const double o = __shfl_up(inc, off, kWave);
+      inc += lane >= off ? o : 0.0;
+    }
+    uint64_t in = __ballot(lane < kLB && base + inc >= tgt);
+    if (in == 0) in = 1ull << (63 - __builtin_clzll(__ballot(add > 0.0) | 1ull));  // lost to rounding: the last one
+    const int k = __builtin_ctzll(in);
+    *before = base + (k > 0 ? __shfl(inc, k - 1, kWave) : 0.0);
+    return L * kLB + k;
+  }
+  // the first bin at which the cumulative count reaches tgt (>= 1), -1 if none does
+  __device__ int find_count(unsigned tgt, unsigned* before) const {
+    const int lane = threadIdx.x % kWave;
+    const uint64_t hit = __ballot(ic >= tgt);
+    if (hit == 0) return -1;
+    const int L = __builtin_ctzll(hit);
+    const unsigned base = L > 0 ? (unsigned)__shfl((int)ic, L - 1, kWave) : 0u;
+    unsigned inc = lane < kLB ? (unsigned)(sh.hist[L * kLB + lane % kLB] >> kCountShift) : 0u;
+#pragma unroll
+    for (int off = 1; off < kLB; off <<= 1) {
+      const unsigned o = (unsigned)__shfl_up((int)inc, off, kWave);
+      inc += lane >= off ? o : 0u;
+    }
+    const int k = __builtin_ctzll(__ballot(lane < kLB && base + inc >= tgt));
+    *before = base + (k > 0 ? (unsigned)__shfl((int)inc, k - 1, kWave) : 0u);
+    return L * kLB + k;
+  }
+  __device__ unsigned count_above(int bin) const {  // entries of the bins < bin
+    const int lane = threadIdx.x % kWave, L = bin / kLB;
+    unsigned v = lane < bin % kLB ? (unsigned)(sh.hist[L * kLB + lane] >> kCountShift) : 0u;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += (unsigned)__shfl_xor((int)v, off, kWave);
+    return v + (L > 0 ? (unsigned)__shfl((int)ic, L - 1, kWave) : 0u);
+  }
+};
+
+// The block's sum of `tail` from its waves' partial sums (sh.red), after a barrier.
+__device__ __forceinline__ void tail_partials(double tail) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) tail += __shfl_xor(tail, off, kWave);
+  if (threadIdx.x % kWave == 0) sh.red[threadIdx.x / kWave] = tail;
+}
+__device__ __forceinline__ double tail_total() {
+  double t = 0.0;
+#pragma unroll
+  for (int w = 0; w < kTW; ++w) t += sh.red[w];
+  return t;
 }
 
-// Places a collection window from a histogram of part of the row (the sample, or the segments seen
+// One wave: places a collection window from a histogram of part of the row (the sample, or the segments seen
 // so far): the bin where that histogram's own boundary falls (the k_seen-th largest for top-k, the
 // top_p mass point for top-p), widened to about `budget` entries of the next segment; `scale` =
-// entries of the next segment per counted entry.
-__device__ void place_window(Shared& sh, bool use_k, float top_p, double k_seen, double scale, double budget,
-                             int* wlo, int* whi) {
-  constexpr int kBPT = kNB / kT;
-  const int tid = threadIdx.x;
-  double lm = 0.0, lc = 0.0;
-  double bm[kBPT], bc[kBPT];
-  double sc = bin_scale(tid * kBPT);
+// entries of the next segment per counted entry. `tail`: the mass below the histogram.
+// The floor (in: the bins below it are counted completely) moves up to just below where the boundary of the
+// whole row can lie, with f = the share of the row seen: for top-k, past the bin by which the count seen exceeds
+// k f by 5 standard deviations; for top-p, where the mass below (seen / f) has shrunk to 3/4 of (1 - top_p) Z for
+// a low estimate of Z, each group of 32 bins scaled up from its count less 3 standard deviations, and below at
+// least 64 counted entries: the few likely tokens of a peaked row lie anywhere above. A floor that proves too
+// high costs the row a second pass. The top (top-p): the bins that hold the row's first kTopCount entries or so.
+// Leaves wlo, whi, top and the floor in sh.ipar[0..3].
+__device__ __forceinline__ void place_window(LaneBins& lb, bool use_k, float top_p, int top_k, float f, double tail,
+                                             float scale, float budget, int floor_bin) {
+  lb.load();
+  const float up = __builtin_amdgcn_rcpf(f);
+  // a low estimate of the row's mass (no entry: 1 - 3 inf = -inf, so a factor of 1)
+  double z_lo = lb.m * (double)fmaxf(1.f, up * (1.f - 3.f * __builtin_amdgcn_rsqf((float)lb.c)));
 #pragma unroll
-  for (int u = 0; u < kBPT; ++u) {
-    const unsigned long long h = sh.hist[tid * kBPT + u];
-    bc[u] = (double)(h >> kCountShift);
-    bm[u] = (double)(float)bin_mass(h, sc);
-    sc *= kBinRatio;
-    lm += bm[u];
-    lc += bc[u];
+  for (int off = 32; off > 0; off >>= 1) z_lo += __shfl_xor(z_lo, off, kWave);
+  z_lo += tail * (double)fmaxf(1.f, 0.9f * up);
+  const double zall = lb.mass() + tail;
+  const float all = budget * __builtin_amdgcn_rcpf(scale), k_seen = (float)top_k * f;  // in counted entries
+  unsigned before = 0u;
+  double mb;
+  int B, wlo = 0, top = 0, fl;
+  float hi_c = all;
+  if (use_k) {
+    B = lb.find_count((unsigned)fmaxf(1.f, ceilf(k_seen)), &before);
+    if (B < 0) B = kNB - 1;
+    const int b = lb.find_count((unsigned)(k_seen + 5.f * __builtin_amdgcn_sqrtf(k_seen) + 12.f), &before);
+    fl = b < 0 ? kNB : b + 3;
+  } else {
+    B = lb.find_mass((double)top_p * zall, &mb);
+    if (B < 0) B = kNB - 1;
+    const int b = lb.find_mass(zall - (double)(0.75f * f * (1.f - top_p)) * z_lo, &mb);
+    const int sparse = lb.find_count((unsigned)(64.f + 512.f * f) + 1u, &before);
+    fl = b < 0 || sparse < 0 ? kNB : max(b + 3, sparse + 1);
+    top = max(lb.find_count((unsigned)((float)kTopCount * f) + 1u, &before), 0);
+    const float cB = (float)lb.count_above(B), nB = (float)(sh.hist[B] >> kCountShift);
+    if (cB - 0.5f * all >= 0.f) wlo = min(max(lb.find_count((unsigned)(cB - 0.5f * all) + 1u, &before), 0), B);
+    hi_c = cB + nB + 0.5f * all;
   }
-  double zb = 0.0, cbins = 0.0;
-  const double exm = block_excl_scan(lm, sh.red, &zb);
-  const double exc = block_excl_scan(lc, sh.red, &cbins);
-  if (tid == 0) {
-    sh.ipar[0] = INT_MAX;
-    sh.ipar[1] = INT_MAX;
-    sh.ipar[2] = -1;
+  int whi = lb.find_count((unsigned)fmaxf(1.f, ceilf(hi_c)), &before);
+  if (whi < 0) whi = kNB - 1;
+  if (threadIdx.x == 0) {
+    sh.ipar[0] = wlo;
+    sh.ipar[1] = min(max(whi, B) + 1, kNB - 1);  // one bin of slack below: values tied across a bin edge
+    sh.ipar[2] = top;
+    sh.ipar[3] = min(floor_bin, fl);
   }
-  __syncthreads();
-  const double tgt = use_k ? k_seen : (double)top_p * (zb + bin_mass(sh.hist[kNB], bin_scale(kNB)));
-  double run = use_k ? exc : exm;
-#pragma unroll
-  for (int u = 0; u < kBPT; ++u) {
-    const double add = pick(use_k, bc[u], bm[u]);
-    if (run < tgt && run + add >= tgt) atomicMin(&sh.ipar[0], tid * kBPT + u);
-    run += add;
+}
+
+// One wave: the mass of the whole row (sh.dpar[0]) and the bin that holds the k-th largest value (top-k) or
+// the nucleus boundary (top-p): sh.ipar[0], -1 if it lies below the histogram; the entries of it and the next bin (top-k:
+// and of all above), sh.ipar[1]; the mass above it, sh.dpar[1].
+__device__ __forceinline__ void find_boundary(LaneBins& lb, bool use_k, float top_p, int top_k, double tail) {
+  lb.load();
+  const double Z = lb.mass() + tail + bin_mass(sh.hist[kNB], bin_scale(kNB));
+  unsigned before = 0u;
+  double mb = 0.0;
+  const int B = use_k ? lb.find_count((unsigned)top_k, &before) : lb.find_mass((double)top_p * Z, &mb);
+  if (threadIdx.x == 0) {
+    unsigned need = before;
+    if (B >= 0)
+      for (int b = B; b <= min(B + 1, kNB - 1); ++b) need += (unsigned)(sh.hist[b] >> kCountShift);
+    sh.ipar[0] = B;
+    sh.ipar[1] = (int)need;
+    sh.dpar[0] = Z;
+    sh.dpar[1] = mb;
   }
-  __syncthreads();
-  int B = sh.ipar[0];
-  if (B == INT_MAX) B = kNB - 1;
-  if (tid == B / kBPT) {
-    double c = exc;
-#pragma unroll
-    for (int u = 0; u < kBPT; ++u) c += u < B % kBPT ? bc[u] : 0.0;  // unrolled: bc stays in registers
-    sh.dpar[1] = c;                                                 // count above B
-    sh.dpar[2] = (double)(sh.hist[B] >> kCountShift);                // count in B
-  }
-  __syncthreads();
-  const double cB = sh.dpar[1], nB = sh.dpar[2];
-  const double half = budget / scale / 2.0;  // in counted entries
-  const double lo_c = use_k ? -1.0 : cB - half, hi_c = use_k ? budget / scale : cB + nB + half;
-  // the first bin whose cumulative count passes lo_c and the last one that starts below hi_c: the
-  // cumulative count (exact in fp64) only grows with the bin, so one bin of each test sees the
-  // transition and a single atomic per test lands (same-address LDS atomics serialise)
-  double c = exc;
-#pragma unroll
-  for (int u = 0; u < kBPT; ++u) {
-    const int bin = tid * kBPT + u;
-    if (c + bc[u] > lo_c && (bin == 0 || c <= lo_c)) atomicMin(&sh.ipar[1], bin);
-    if (c < hi_c && (bin == kNB - 1 || c + bc[u] >= hi_c)) atomicMax(&sh.ipar[2], bin);
-    c += bc[u];
-  }
-  __syncthreads();
-  *wlo = use_k ? 0 : min(sh.ipar[1], B);
-  *whi = min(max(sh.ipar[2], B) + 1, kNB - 1);  // one bin of slack below: values tied across a bin edge
-  __syncthreads();
 }
 
 // Exact y = x / T of the collected logits, in place.
 template <bool kDiv>
-__device__ void collected_to_y(Shared& sh, int n, double rt) {
+__device__ void collected_to_y(int n, double rt) {
   for (int j = threadIdx.x; j < n; j += kT) sh.coll[j] = exact_y<kDiv>(sh.coll[j], rt);
   __syncthreads();
 }
 
 // Top-p candidates (the collected logits of the boundary bin B and of bin B + 1) to exact y, in place,
-// packed at the front; returns how many. Bins are monotone in the logit, so a value of bin B + 1 is
-// <= every value of bin B in y and can only be kept when it ties with the smallest of them: the
-// others are dropped, which about halves what is sorted.
+// packed at the front; returns how many, and the largest and smallest. Bins are monotone in the logit, so a value
+// of bin B + 1 is <= every value of bin B in y and can only be kept when it ties with the smallest of them: the
+// others are dropped, which about halves what is looked at.
 template <bool kDiv>
-__device__ int boundary_to_y(Shared& sh, const BinMap& bm, int n, int B, double rt) {
-  constexpr int kPer = kCap / kT;
+__device__ __forceinline__ int boundary_to_y(const BinMap& bm, int n, int B, double rt, float* ytop, float* ylow) {
+  constexpr int kPer = kSortCap / kT;
   float y[kPer];
   unsigned inb = 0u;  // bit u: entry u is in bin B (then: is kept)
-  float ymin = INFINITY;
+  float ymin = INFINITY, ymax = -INFINITY;
 #pragma unroll
   for (int u = 0; u < kPer; ++u) {
-    const int j = (int)threadIdx.x * kPer + u;
+    if (u * kT >= n) break;  // block-uniform
+    const int j = u * kT + (int)threadIdx.x;
     const float x = j < n ? sh.coll[j] : -INFINITY;
     const bool in = j < n && (int)bm.bin(x) == B;
     y[u] = j < n ? exact_y<kDiv>(x, rt) : -INFINITY;
     ymin = in ? fminf(ymin, y[u]) : ymin;
+    ymax = in ? fmaxf(ymax, y[u]) : ymax;
     inb |= (unsigned)in << u;
   }
-  ymin = -block_max(-ymin, sh.red);
-  const int nl = max(min(n - (int)threadIdx.x * kPer, kPer), 0);  // this thread's entries
+  ymin = -block_max(-ymin);
+  ymax = block_max(ymax);
 #pragma unroll
-  for (int u = 0; u < kPer; ++u) inb |= (unsigned)(u < nl && y[u] == ymin) << u;
+  for (int u = 0; u < kPer; ++u) {
+    if (u * kT >= n) break;
+    inb |= (unsigned)(u * kT + (int)threadIdx.x < n && y[u] == ymin) << u;
+  }
   double tot = 0.0;
-  int w = (int)block_excl_scan((double)__popc(inb), sh.red, &tot);  // every read of sh.coll precedes its barriers
+  int w = (int)block_excl_scan((double)__popc(inb), &tot);  // every read of sh.coll precedes its barriers
 #pragma unroll
   for (int u = 0; u < kPer; ++u)
     if ((inb >> u) & 1u) sh.coll[w++] = y[u];
   __syncthreads();
+  *ytop = ymax;
+  *ylow = ymin;
   return (int)tot;
 }
 
-template <bool kDiv, bool kVec>
+// The nucleus boundary among the n values y of sh.coll (ylow <= y <= ytop, within a bin): the smallest y whose
+// strictly preceding mass (descending) is below tgt, masses exp(y - ytop). A histogram of kSub sub-bins finds the
+// one that crosses tgt, and one wave ranks its few values against each other (a bitonic sort of all of
+// them took a quarter of the kernel's instructions). *mass: the mass of every value >= thr. Masses are summed as
+// integers, 46 bits below ytop's: the result does not depend on the order. False (nothing done to sh.coll) when
+// the sub-bin holds more than a wave's values.
+__device__ __forceinline__ bool sub_boundary(int n, float ytop, float ylow, double tgt, float* thr, double* mass) {
+  const int tid = threadIdx.x;
+  unsigned long long* sub = sh.hist;
+  const double tq = tgt * 0x1p46;
+  if (!(tq > 0.0) || !(ytop > ylow)) {  // the largest value alone, with its ties
+    const float t = ytop > ylow ? ytop : ylow;
+    double c = 0.0;
+    for (int j = tid; j < n; j += kT) c += sh.coll[j] == t;
+    *thr = t;
+    *mass = block_sum(c);
+    return true;
+  }
+  const float inv = (float)kSub / (ytop - ylow);
+  auto sub_of = [&](float y) { return min(kSub - 1, (int)((ytop - y) * inv)); };
+  auto mass_of = [&](float y) { return (unsigned long long)(exp((double)y - (double)ytop) * 0x1p46); };
+  __syncthreads();  // the histogram has been read
+  for (int j = tid; j < kSub; j += kT) sub[j] = 0ull;
+  if (tid == 0) sh.n = 0;
+  __syncthreads();
+  for (int j = tid; j < n; j += kT) atomicAdd(&sub[sub_of(sh.coll[j])], mass_of(sh.coll[j]));
+  __syncthreads();
+  if (tid < kWave) {
+    constexpr int kPL = kSub / kWave;
+    unsigned long long s = 0ull;
+#pragma unroll 4
+    for (int i = 0; i < kPL; ++i) s += sub[tid * kPL + (tid + i) % kPL];
+    unsigned long long inc = s;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const unsigned long long o = __shfl_up(inc, off, kWave);
+      inc += tid >= off ? o : 0ull;
+    }
+    const uint64_t hit = __ballot((double)inc >= tq);
+    if (hit == 0) {
+      if (tid == 0) sh.ipar[0] = -1;
+      if (tid == kWave - 1) sh.dpar[0] = (double)inc;
+    } else if (tid == (int)__builtin_ctzll(hit)) {
+      unsigned long long run = inc - s;
+      int i = 0;
+      while (i < kPL - 1 && (double)(run + sub[tid * kPL + i]) < tq) run += sub[tid * kPL + i++];
+      sh.ipar[0] = tid * kPL + i;
+      sh.dpar[0] = (double)run;
+    }
+  }
+  __syncthreads();
+  const int S = sh.ipar[0];
+  const double above = sh.dpar[0];
+  if (S < 0) {  // tgt exceeds the sum (by rounding): every value is kept
+    *thr = ylow;
+    *mass = above * 0x1p-46;
+    return true;
+  }
+  float* list = sh.queue[0];
+  for (int j = tid; j < n; j += kT) {
+    const float y = sh.coll[j];
+    if (sub_of(y) == S) {
+      const int at = atomicAdd(&sh.n, 1);
+      if (at < kWave) list[at] = y;
+    }
+  }
+  __syncthreads();
+  const int cnt = sh.n;
+  if (cnt > kWave) return false;
+  if (tid < kWave) {
+    const float y = tid < cnt ? list[tid] : -INFINITY;
+    const unsigned long long q = tid < cnt ? mass_of(y) : 0ull;
+    unsigned long long prec = 0ull;  // the mass of the list's values before this one (ties in list order)
+    for (int j = 0; j < cnt; ++j) {
+      const float yj = __shfl(y, j, kWave);
+      const unsigned long long qj = __shfl(q, j, kWave);
+      prec += yj > y || (yj == y && j < tid) ? qj : 0ull;
+    }
+    const bool kept = tid < cnt && above + (double)prec < tq;
+    float t = kept ? y : INFINITY;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) t = fminf(t, __shfl_xor(t, off, kWave));
+    if (t == INFINITY) t = wave_max(y);  // (cannot be: the sub-bin's first value starts below tgt)
+    unsigned long long at = tid < cnt && y >= t ? q : 0ull;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) at += __shfl_xor(at, off, kWave);
+    if (tid == 0) {
+      sh.dpar[1] = above + (double)at;
+      sh.dpar[2] = (double)t;
+    }
+  }
+  __syncthreads();
+  *thr = (float)sh.dpar[2];
+  *mass = sh.dpar[1] * 0x1p-46;
+  return true;
+}
+
+template <bool kDiv>
 __global__ __launch_bounds__(kT, 4) void truncate_kernel(TruncArgs a) {
-  __shared__ Shared sh;
   const int b = blockIdx.x / a.G, i = a.first + (int)(blockIdx.x % a.G);
   if (i >= a.R || (a.state && a.state[b] >= 0)) return;  // block-uniform: past the rows, or decided
   const int r = b * a.R + i;
-  const float* row = a.logits + (int64_t)b * a.batch_stride + (int64_t)i * a.row_stride;
   const int V = a.V, tid = threadIdx.x;
+  const RowView rv(a.logits + (int64_t)b * a.batch_stride + (int64_t)i * a.row_stride, V);
   const bool use_k = a.top_k > 0 && a.top_k < V;
   const bool use_p = a.top_p < 1.f;
   const bool collect = use_k || use_p;
@@ -752,7 +1035,9 @@ __global__ __launch_bounds__(kT, 4) void truncate_kernel(TruncArgs a) {
   int passes = 0;  // segments streamed (kSeg = one pass over the row)
 
   float mx = -INFINITY;  // max logit (the banned id excluded)
-  unsigned nanbits = 0u;
+  bool nan = false;
+  double Z = 0.0, cum = 0.0;  // window path: the row's mass and the mass above the boundary bin
+  int B = -1, need = 0;       // the boundary bin and the entries it takes to resolve it
   float mref = 0.f;
   BinMap bm{};
   if (window) {
@@ -761,16 +1046,16 @@ __global__ __launch_bounds__(kT, 4) void truncate_kernel(TruncArgs a) {
     const int ns = min(kSample, V);
     float xs[kSample / kT];
     float smax = -INFINITY;
-    if (kVec && V >= 4 * kSample) {
+    if (rv.n4 >= kSample) {
       // kT evenly spaced 16-byte vectors of 4 adjacent entries each: a line per 4 entries (entries one
       // by one would fetch a line each, a quarter of the row's bytes at V = 248320)
       static_assert(kSample == 4 * kT, "one vector of the sample per thread");
-      const int jv = (int)((int64_t)tid * (V >> 2) / kT);
-      const u32x4 w = reinterpret_cast<const u32x4*>(row)[jv];
+      const int jv = (int)((int64_t)tid * rv.n4 / kT);
+      const u32x4 w = rv.body[jv];
       const float x4[4] = {__uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z), __uint_as_float(w.w)};
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        xs[u] = (4 * jv + u != a.ban && x4[u] == x4[u]) ? x4[u] : -INFINITY;
+        xs[u] = (rv.pre + 4 * jv + u != a.ban && x4[u] == x4[u]) ? x4[u] : -INFINITY;
         smax = xs[u] < INFINITY ? fmaxf(smax, xs[u]) : smax;
       }
     } else {
@@ -778,78 +1063,99 @@ __global__ __launch_bounds__(kT, 4) void truncate_kernel(TruncArgs a) {
       for (int u = 0; u < kSample / kT; ++u) {
         const int j = u * kT + tid;
         const int ix = (int)((int64_t)min(j, ns - 1) * V / ns);
-        const float x = row[ix];
+        const float x = rv.row[ix];
         xs[u] = (j < ns && ix != a.ban && x == x) ? x : -INFINITY;
         smax = xs[u] < INFINITY ? fmaxf(smax, xs[u]) : smax;
       }
     }
-    smax = block_max(smax, sh.red);
-    mref = smax > -INFINITY ? exact_y<kDiv>(smax, a.rt) : 0.f;
-    const float rf = (float)a.rt;
-    bm.tA = -kPerNat * rf;
-    bm.tB = kPerNat * (kTop + mref);
-    bm.rf = rf;
-    bm.nm = -mref;
     for (int j = tid; j <= kNB; j += kT) sh.hist[j] = 0ull;
-    __syncthreads();
-    int w_lo = kNB + 1, w_hi = kNB + 1;  // empty
+    smax = block_max(smax);
+    mref = smax > -INFINITY ? exact_y<kDiv>(smax, a.rt) : 0.f;
+    bm.set(a.rt, mref);
+    LaneBins lb;
+    if (tid < kWave) lb.init();
     if (collect) {
 #pragma unroll
       for (int u = 0; u < kSample / kT; ++u) {
         const float x = xs[u] < INFINITY ? xs[u] : -INFINITY;
         const unsigned bin = bm.bin(x);
-        const float d = fmaf(x, bm.rf, bm.nm);
-        const float top = fmaf((float)bin, -1.f / kPerNat, kTop);
-        const float rr = __builtin_amdgcn_exp2f(fmaf(d - top, 1.44269504f, 26.f));
-        atomicAdd(&sh.hist[bin], (1ull << kCountShift) | (unsigned long long)(unsigned)rr);
+        if (bin < (unsigned)kNB) atomicAdd(&sh.hist[bin], bm.packed(x, bin));
       }
-      __syncthreads();
-      int s0, s1;
-      seg_bounds<kVec>(V, 0, &s0, &s1);
-      place_window(sh, use_k, a.top_p, (double)a.top_k * ns / V, (double)(s1 - s0) / ns, 0.2 * kCap, &w_lo, &w_hi);
-      for (int j = tid; j <= kNB; j += kT) sh.hist[j] = 0ull;
     }
     if (tid == 0) sh.n = 0;
     __syncthreads();
-
-    // ---- the streaming pass, kSeg segments: max, histogram, collection of a window re-placed from the
-    // exact histogram after every segment
-    for (int s = 0; s < kSeg; ++s) {
-      int e0, e1;
-      seg_bounds<kVec>(V, s, &e0, &e1);
-      if (tid == 0) {
-        sh.wlo[s] = w_lo;
-        sh.whi[s] = w_hi;
-      }
-      stream_segment<kVec, true>(row, a, bm, e0, e1, w_lo, w_hi, sh, mx, nanbits);
-      ++passes;
-      __syncthreads();
-      if (tid == 0) sh.nseg[s] = sh.n;
-      if (collect && s + 1 < kSeg) {
+    // ---- the streaming pass, kSeg segments: max, histogram down to the floor, collection of a window placed
+    // from the sample's histogram and again from the row's own after every segment. Run again without
+    // floors when the boundary turns out to lie below the last one.
+    int w_lo = kNB + 1, w_hi = kNB + 1, w_top = 0, floor_bin = collect ? kNB : 0;
+    int seen = 0, counted = ns;
+    double tail = 0.0;
+    bool floors = true;
+    int s = collect ? -1 : 0;
+    while (true) {
+      if (s >= 0) {
+        if (tid == 0) {
+          sh.wlo[s] = w_lo;
+          sh.whi[s] = min(w_hi, floor_bin - 1);
+          sh.top[s] = min(w_top, floor_bin);
+        }
+        stream_segment<true>(rv, a, bm, s, collect ? below_bin(bm, floor_bin) : INFINITY, 0.f, w_top, w_lo, w_hi, mx, tail);
+        ++passes;
+        seen += seg_size(rv, s);
+        counted = seen;
+        tail_partials(tail);
         __syncthreads();
-        int n0, n1;
-        seg_bounds<kVec>(V, s + 1, &n0, &n1);
-        const double seen = (double)e1, next = (double)(n1 - n0);
-        const double room = max(0.6 * kCap - (double)min(sh.n, kCap), 0.0);
-        place_window(sh, use_k, a.top_p, (double)a.top_k * seen / V, next / seen, room / (kSeg - 1 - s), &w_lo,
-                     &w_hi);
+        if (tid == 0) sh.nseg[s] = sh.n;
       }
+      const int next = s + 1 < kSeg ? seg_size(rv, s + 1) : 0;
+      if (s == kSeg - 1) {
+        if (tid < kWave) find_boundary(lb, use_k, a.top_p, a.top_k, tail_total() * bm.cold_scale);
+      } else if (collect && next > 0 && tid < kWave) {
+        const float room = fmaxf(0.75f * kCap - (float)min(sh.n, kCap), 0.f);
+        place_window(lb, use_k, a.top_p, a.top_k, (float)counted / (float)V, s < 0 ? 0.0 : tail_total() * bm.cold_scale,
+                     (float)next / (float)counted, s < 0 ? 0.2f * kCap : room / (float)(kSeg - 1 - s), floor_bin);
+      }
+      __syncthreads();
+      if (s == kSeg - 1) {
+        B = sh.ipar[0];
+        need = sh.ipar[1];
+        Z = sh.dpar[0];
+        cum = sh.dpar[1];
+        // the boundary bin and the one below it have to lie above the floor
+        if (!collect || floor_bin >= kNB || (B >= 0 && B + 1 < floor_bin)) break;
+        floors = false;
+        floor_bin = kNB;
+        tail = 0.0;
+        seen = 0;
+        s = -1;  // the last window stands for the first segment
+        __syncthreads();
+        for (int j = tid; j <= kNB; j += kT) sh.hist[j] = 0ull;
+        if (tid == 0) sh.n = 0;
+      } else if (collect && next > 0) {
+        w_lo = sh.ipar[0];
+        w_hi = sh.ipar[1];
+        w_top = sh.ipar[2];
+        if (floors && s >= 0) floor_bin = sh.ipar[3];
+        if (s < 0)
+          for (int j = tid; j <= kNB; j += kT) sh.hist[j] = 0ull;
+      }
+      __syncthreads();
+      ++s;
     }
+    nan = tail != tail;
   } else {
-    for_each_y<kDiv, kVec>(row, V, a.rt, a.ban, [&](float y, int ix, bool ok) {
+    for_each_y<kDiv>(rv, a.rt, a.ban, [&](float y, int ix, bool ok) {
       mx = fmaxf(mx, ok ? y : -INFINITY);
-      nanbits = max(nanbits, ok ? __float_as_uint(y) << 1 : 0u);
+      nan |= ok && y != y;
     });
     passes += kSeg;
   }
-  mx = block_max(mx, sh.red);
+  mx = block_max(mx);
   if (tid == 0) sh.umax = 0u;
   __syncthreads();
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) nanbits = max(nanbits, (unsigned)__shfl_xor((int)nanbits, off, kWave));
-  if (tid % kWave == 0) atomicMax(&sh.umax, nanbits);  // one atomic per wave
+  if (__ballot(nan) && tid % kWave == 0) atomicOr(&sh.umax, 1u);
   __syncthreads();
-  const bool bad = sh.umax > 0xff000000u || mx == INFINITY;  // a NaN, or a +inf logit
+  const bool bad = sh.umax != 0u || mx == INFINITY;  // a NaN, or a +inf logit
   // the exact row max of y (the window path tracked the raw logits; y = x / T is monotone in x)
   const float ymax = window ? exact_y<kDiv>(mx, a.rt) : mx;
   float thr = -INFINITY;
@@ -860,111 +1166,67 @@ __global__ __launch_bounds__(kT, 4) void truncate_kernel(TruncArgs a) {
   } else if (!(ymax > -INFINITY)) {
     status = 2;
   } else {
-    bool ok = window && !(ymax - mref > kTop);
-    const int n = sh.n;
     const double md = (double)ymax;
-    const double scale = exp((double)mref - md);
-    if (ok) {
-      // each thread owns kNB / kT consecutive bins; exclusive scans give the mass / count above each
-      constexpr int kBPT = kNB / kT;
-      double lm = 0.0, lc = 0.0;
-      double bms[kBPT], bcs[kBPT];
-      double sc = bin_scale(tid * kBPT);
-#pragma unroll
-      for (int u = 0; u < kBPT; ++u) {
-        const unsigned long long h = sh.hist[tid * kBPT + u];
-        bcs[u] = (double)(h >> kCountShift);
-        bms[u] = bin_mass(h, sc);
-        sc *= kBinRatio;
-        lm += bms[u];
-        lc += bcs[u];
+    // the target must lie within the histogram, and what resolves it fit the collection
+    bool ok = window && !(ymax - mref > kTop) && (!collect || (B >= 0 && need <= kSortCap));
+    if (ok && !collect) {
+      zk = Z * exp((double)mref - md);
+    } else if (ok) {
+      // values tied in y may straddle a bin edge (the bins come from the logits), so the
+      // candidate set takes one more bin below the boundary bin
+      const int c_lo = use_k ? 0 : B, c_hi = min(B + 1, kNB - 1);
+      // keep what the segments whose window held [c_lo, c_hi] collected (and that fit the
+      // collection); stream the others again
+      unsigned complete = 0u;
+      for (int s = 0; s < kSeg; ++s)
+        complete |= (unsigned)(((c_lo >= sh.wlo[s] && c_hi <= sh.whi[s]) || c_hi < sh.top[s]) && sh.nseg[s] <= kCap) << s;
+      int n2 = compact_bins(bm, min(sh.n, kCap), c_lo, c_hi, complete);
+      if (complete != (1u << kSeg) - 1u) {
+        __syncthreads();
+        if (tid == 0) sh.n = n2;
+        __syncthreads();
+        const float x_lo = below_bin(bm, c_hi + 1), x_hi = c_lo > 1 ? below_bin(bm, c_lo - 2) : INFINITY;
+        double none = 0.0;
+        for (int s = 0; s < kSeg; ++s) {
+          if ((complete >> s) & 1u) continue;
+          stream_segment<false>(rv, a, bm, s, x_lo, x_hi, 0, c_lo, c_hi, mx, none);
+          ++passes;
+        }
+        __syncthreads();
+        n2 = min(sh.n, kSortCap);
       }
-      double zb = 0.0, cbins = 0.0;
-      const double exm = block_excl_scan(lm, sh.red, &zb);
-      const double exc = block_excl_scan(lc, sh.red, &cbins);
-      const double Z = zb + bin_mass(sh.hist[kNB], bin_scale(kNB));
-      if (!collect) {
-        zk = Z * scale;
+      if (use_k) {
+        collected_to_y<kDiv>(n2, a.rt);
+        sort_collection(n2);
+        const int k = min(a.top_k, n2);
+        thr = sh.coll[k - 1];
+        if (use_p) {
+          double Sk = 0.0, tot = 0.0;
+          (void)count_below(k, md, 0.0, -1.0, &Sk);
+          const int nk = max(count_below(k, md, 0.0, (double)a.top_p * Sk, &tot), 1);
+          thr = sh.coll[nk - 1];
+        }
+        zk = mass_at_least(n2, thr, md);
       } else {
-        // the bin holding the k-th largest value (top-k) or the nucleus boundary (top-p)
-        const double tgt = use_k ? (double)a.top_k : (double)a.top_p * Z;
-        if (tid == 0) sh.ipar[0] = INT_MAX;
-        __syncthreads();
-        double run = use_k ? exc : exm;
-#pragma unroll
-        for (int u = 0; u < kBPT; ++u) {
-          const double add = pick(use_k, bcs[u], bms[u]);
-          if (run < tgt && run + add >= tgt) atomicMin(&sh.ipar[0], tid * kBPT + u);
-          run += add;
-        }
-        __syncthreads();
-        const int B = sh.ipar[0];
-        if (B != INT_MAX && tid == B / kBPT) {  // the owner publishes the count / mass above the bin
-          double cum = use_k ? exc : exm;
-#pragma unroll
-          for (int u = 0; u < kBPT; ++u) cum += u < B % kBPT ? pick(use_k, bcs[u], bms[u]) : 0.0;
-          sh.dpar[0] = cum;
-        }
-        __syncthreads();
-        if (B == INT_MAX) {
-          ok = false;  // the target lies below the histogram's range
+        float ytop, ylow;
+        n2 = boundary_to_y<kDiv>(bm, n2, B, a.rt, &ytop, &ylow);
+        const double base = cum * exp((double)mref - md), target = (double)a.top_p * Z;
+        const double et = exp((double)ytop - md);
+        double mass;
+        if (sub_boundary(n2, ytop, ylow, (target - cum) * exp((double)mref - (double)ytop), &thr, &mass)) {
+          zk = base + mass * et;
         } else {
-          // values tied in y may straddle a bin edge (the bins come from the logits), so the
-          // candidate set takes one more bin below the boundary bin
-          const double cum = sh.dpar[0];
-          const int c_lo = use_k ? 0 : B, c_hi = min(B + 1, kNB - 1);
-          double need = use_k ? cum : 0.0;
-          for (int bb = B; bb <= c_hi; ++bb) need += (double)(sh.hist[bb] >> kCountShift);
-          if (need > kCap) {
-            ok = false;
-          } else {
-            // keep what the segments whose window held [c_lo, c_hi] collected (and that fit the
-            // collection); stream the others again
-            unsigned complete = 0u;
-            for (int s = 0; s < kSeg; ++s)
-              complete |= (unsigned)(c_lo >= sh.wlo[s] && c_hi <= sh.whi[s] && sh.nseg[s] <= kCap) << s;
-            int n2 = compact_bins(sh, bm, min(n, kCap), c_lo, c_hi, complete);
-            __syncthreads();
-            if (tid == 0) sh.n = n2;
-            __syncthreads();
-            for (int s = 0; s < kSeg; ++s) {
-              if ((complete >> s) & 1u) continue;
-              int e0, e1;
-              seg_bounds<kVec>(V, s, &e0, &e1);
-              stream_segment<kVec, false>(row, a, bm, e0, e1, c_lo, c_hi, sh, mx, nanbits);
-              ++passes;
-            }
-            __syncthreads();
-            n2 = min(sh.n, kCap);
-            if (use_k)
-              collected_to_y<kDiv>(sh, n2, a.rt);
-            else
-              n2 = boundary_to_y<kDiv>(sh, bm, n2, B, a.rt);
-            sort_collection(sh, n2);
-            if (use_k) {
-              const int k = min(a.top_k, n2);
-              thr = sh.coll[k - 1];
-              if (use_p) {
-                double Sk = 0.0, tot = 0.0;
-                (void)count_below(sh.coll, k, md, 0.0, -1.0, &Sk, sh.red);
-                const int nk = max(count_below(sh.coll, k, md, 0.0, (double)a.top_p * Sk, &tot, sh.red), 1);
-                thr = sh.coll[nk - 1];
-              }
-              zk = mass_at_least(sh.coll, n2, thr, md, sh.red);
-            } else {
-              const double base = cum * scale, target = tgt * scale;
-              double tot = 0.0;
-              const int nk = min(max(count_below(sh.coll, n2, md, base, target, &tot, sh.red), 1), max(n2, 1));
-              thr = sh.coll[nk - 1];
-              zk = base + mass_at_least(sh.coll, n2, thr, md, sh.red);
-            }
-          }
+          sort_collection(n2);
+          double tot = 0.0;
+          const int nk = min(max(count_below(n2, md, base, target * exp((double)mref - md), &tot), 1), max(n2, 1));
+          thr = sh.coll[nk - 1];
+          zk = base + mass_at_least(n2, thr, md);
         }
       }
     }
     if (!ok) {
       int rp = 0;
-      radix_resolve<kDiv, kVec>(row, a, ymax, use_k, use_p, sh, &thr, &zk, &rp);
+      radix_resolve<kDiv>(rv, a, ymax, use_k, use_p, &thr, &zk, &rp);
       passes += rp * kSeg;
     }
   }
@@ -1226,16 +1488,9 @@ __global__ __launch_bounds__(kRT) void resid_pick_kernel(AcceptArgs a) {
 
 int ban_of(int64_t ban_id, int64_t V) { return (ban_id >= 0 && ban_id < V) ? (int)ban_id : -1; }
 
-bool vec_ok(const void* p, int64_t V, int64_t bs, int64_t rs) {
-  return ((uintptr_t)p % 16 == 0) && V % 4 == 0 && bs % 4 == 0 && rs % 4 == 0;
-}
-
-int launch_truncate(const TruncArgs& ta, int rows, bool vec, hipStream_t st) {
-  const bool div = ta.rt != 1.0;
-  if (div && vec) hipLaunchKernelGGL((truncate_kernel<true, true>), dim3(rows), dim3(kT), 0, st, ta);
-  else if (div) hipLaunchKernelGGL((truncate_kernel<true, false>), dim3(rows), dim3(kT), 0, st, ta);
-  else if (vec) hipLaunchKernelGGL((truncate_kernel<false, true>), dim3(rows), dim3(kT), 0, st, ta);
-  else hipLaunchKernelGGL((truncate_kernel<false, false>), dim3(rows), dim3(kT), 0, st, ta);
+int launch_truncate(const TruncArgs& ta, int rows, hipStream_t st) {
+  if (ta.rt != 1.0) hipLaunchKernelGGL((truncate_kernel<true>), dim3(rows), dim3(kT), 0, st, ta);
+  else hipLaunchKernelGGL((truncate_kernel<false>), dim3(rows), dim3(kT), 0, st, ta);
   return launch_status("truncate_kernel");
 }
 
@@ -1295,8 +1550,7 @@ extern "C" int trida_truncate_stats(const float* logits, int64_t B, int64_t R, i
   TruncArgs ta{logits, batch_stride, row_stride, (int)R, (int)V, 1.0 / (double)temperature, (int)top_k, top_p,
                ban_of(ban_id, V), flags, (int)R, 0, nullptr,
                m_out, thr_out, zk_out, status_out, passes_out};
-  return launch_truncate(ta, (int)(B * R), vec_ok(logits, V, batch_stride, row_stride),
-                         static_cast<hipStream_t>(stream));
+  return launch_truncate(ta, (int)(B * R), static_cast<hipStream_t>(stream));
 }
 
 extern "C" int64_t trida_sample_accept_scratch_bytes(int64_t B, int64_t R, int64_t V, int64_t K) {
@@ -1352,14 +1606,13 @@ extern "C" int trida_sample_accept(const float* p_logits, int64_t B, int64_t R, 
   // of the rest at once (decided sequences' blocks exit at once), followed by the final scan.
   const int R1 = (int)K + 1;
   const int G0 = (int)std::min<int64_t>(R1, std::max<int64_t>(8, cdiv(512, B)));
-  const bool vec = vec_ok(p_logits, V, p_batch_stride, p_row_stride);
   int r = TRIDA_OK;
   for (int g = 0; g < 2; ++g) {
     const int first = g == 0 ? 0 : G0, cnt = g == 0 ? G0 : R1 - G0;
     if (cnt <= 0) break;
     TruncArgs ta{p_logits, p_batch_stride, p_row_stride, R1, (int)V, 1.0 / (double)temperature, (int)top_k, top_p,
                  ban_of(ban_id, V), 0, cnt, first, g > 0 ? state : nullptr, m, thr, zk, st, nullptr};
-    r = launch_truncate(ta, (int)(B * cnt), vec, stream);
+    r = launch_truncate(ta, (int)(B * cnt), stream);
     if (r != TRIDA_OK) return r;
     hipLaunchKernelGGL(accept_scan_kernel, dim3(B), dim3(kWave), 0, stream, aa, first, cnt);
     r = launch_status("accept_scan_kernel");

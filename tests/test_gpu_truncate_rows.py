@@ -56,3 +56,35 @@ def test_late_tokens(gpu, T, k, p):
     x[4] = x[4].mul(8).round().div(8)   # massive ties
     x[5] = x[5].mul(0.05)               # a flat row: everything within a few bins
     check(x.view(2, 3, V), T, k, p)
+
+
+@pytest.mark.parametrize("V", [1, 5, 1027, 4 * TILE + 1, 33 * 4096 + 7])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_draw_unaligned_rows(gpu, V, dtype):
+    """The gathered rows, the draws and the probability rows of rows at any offset within a line: exact copies, the
+    inverse CDF of the fp64 distribution outside 1e-6 of a step, probabilities to 4e-6 (the rounding of
+    an fp32 exponent of up to 24, times log2(e))."""
+    g = torch.Generator(device=gpu).manual_seed(V)
+    B, R = 2, 3
+    src = (torch.randn(B, R, V + 3, generator=g, device=gpu) * 3).to(dtype)[..., 1: 1 + V]
+    sel = torch.tensor([[2, 0, 1], [1, 1, 0]], device=gpu)
+    out = torch.full((B, R, V + 2), -7.0, device=gpu)
+    lf = TK.gather_rows(src, sel, out=out[..., 1: 1 + V])
+    assert torch.equal(lf, torch.stack([src[b, sel[b]].float() for b in range(B)]))
+    assert (out[..., 0] == -7).all() and (out[..., -1] == -7).all()
+    stats = TK.truncate_stats(lf, temperature=0.8, top_k=0, top_p=0.9)[:3]
+    u = torch.rand(B * R, generator=g, device=gpu)
+    tok = TK.sample_rows(lf, stats, u, temperature=0.8).view(-1).tolist()
+    q = torch.full((B, R, V + 2), -7.0, device=gpu)
+    rows = torch.arange(R, device=gpu).repeat(B, 1).contiguous()
+    TK.truncated_probs_rows(lf, stats, rows, rows, q[..., 1: 1 + V], temperature=0.8)
+    y = (lf.cpu() / torch.tensor(0.8)).double().to(gpu)  # the CPU's division rounds correctly
+    P = torch.where(y >= stats[1][..., None].double(), torch.exp(y - stats[0][..., None]), torch.zeros_like(y))
+    P = P / P.sum(-1, keepdim=True)
+    torch.testing.assert_close(q[..., 1: 1 + V].double(), P, rtol=4e-6, atol=0)
+    assert (q[..., 0] == -7).all() and (q[..., -1] == -7).all()
+    cdf = P.view(B * R, V).cumsum(-1)
+    for i in range(B * R):
+        lo = cdf[i, tok[i] - 1].item() if tok[i] else 0.0
+        assert lo - 1e-6 <= u[i].item() < cdf[i, tok[i]].item() + 1e-6
+        assert P.view(B * R, V)[i, tok[i]] > 0

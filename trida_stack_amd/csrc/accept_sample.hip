@@ -1286,9 +1286,12 @@ struct RowW {
   float m, thr, inv_zk;
   double rt;
   int ban;
+  __device__ __forceinline__ float prob(float x, int ix) const {
+    const float y = make_y<true>(x, ix, rt, ban);
+    return (y > -INFINITY && y >= thr) ? __expf(y - m) * inv_zk : 0.f;
+  }
   __device__ __forceinline__ void at(int ix, float* w, float* pp) const {
-    const float y = make_y<true>(p[ix], ix, rt, ban);
-    const float P = (y > -INFINITY && y >= thr) ? __expf(y - m) * inv_zk : 0.f;
+    const float P = prob(p[ix], ix);
     *pp = P;
     *w = q ? fmaxf(P - q[ix], 0.f) : P;
   }
@@ -1376,12 +1379,47 @@ __global__ __launch_bounds__(kRT) void resid_sums_kernel(AcceptArgs a) {
   const RowW rw = row_weights(a, b, s_nacc);
   const int lo = c * a.chunk, hi = min(a.V, lo + a.chunk);
   double sw = 0.0, sp = 0.0;
-  for (int ix = lo + tid; ix < hi; ix += kRT) {
-    float w, pp;
-    rw.at(ix, &w, &pp);
-    sw += w;
-    sp += pp;
+  // Four 16-byte loads in flight per thread, the elements outside the chunk's aligned vectors (<= 6) one per thread.
+  // One element per load and iteration left the pass waiting on memory: 512 rows of 248320 185 -> 97 us
+  // (2.7 -> 5.2 TB/s). q is read by element where its rows are not aligned as p's.
+  const float* pc = rw.p + lo;
+  const int len = hi - lo, pre = min((int)((0u - (unsigned)((uintptr_t)pc >> 2)) & 3u), len), n4 = (len - pre) >> 2;
+  const u32x4* p4 = reinterpret_cast<const u32x4*>(pc + pre);
+  const float* qc = rw.q ? rw.q + lo : nullptr;
+  const bool qvec = qc && ((uintptr_t)(qc + pre) & 15) == 0;
+  auto add = [&](float x, float q, int ix) {
+    const float P = rw.prob(x, ix);
+    sp += P;
+    if (qc) sw += fmaxf(P - q, 0.f);
+  };
+  constexpr int U = 4;
+  for (int base = 0; base < n4; base += kRT * U) {
+    u32x4 x[U], qv[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int j = min(base + u * kRT + tid, n4 - 1);
+      x[u] = p4[j];
+      qv[u] = u32x4{0u, 0u, 0u, 0u};
+      if (qvec) {
+        qv[u] = *reinterpret_cast<const u32x4*>(qc + pre + 4 * j);
+      } else if (qc) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) qv[u][e] = __float_as_uint(qc[pre + 4 * j + e]);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int j = base + u * kRT + tid;
+      if (j >= n4) continue;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) add(__uint_as_float(x[u][e]), __uint_as_float(qv[u][e]), lo + pre + 4 * j + e);
+    }
   }
+  {
+    const int j = tid < pre ? tid : tid + 4 * n4;
+    if (j < len) add(pc[j], qc ? qc[j] : 0.f, lo + j);
+  }
+  if (!qc) sw = sp;
   sw = rblock_sum(sw, s_red);
   sp = rblock_sum(sp, s_red);
   if (tid == 0) {
@@ -1400,32 +1438,52 @@ __global__ __launch_bounds__(kRT) void resid_pick_kernel(AcceptArgs a) {
   __shared__ double s_red[kRT / kWave];
   __shared__ float s_w[kPickChunk];
   const int r = a.n_acc[b];
-  if (tid == 0) {
+  // one wave finds the chunk, lane l holding the chunks [l L, l L + L): a serial walk over the chunk sums by one
+  // thread was a memory latency per chunk (512 rows of 61 chunks: 25 -> 17 us)
+  if (tid < kWave) {
     const double* s = a.sums + (int64_t)b * a.NC * 2;
-    double tw = 0.0, tp = 0.0;
-    for (int c = 0; c < a.NC; ++c) {
-      tw += s[2 * c];
-      tp += s[2 * c + 1];
+    const int L = (a.NC + kWave - 1) / kWave, c0 = min(a.NC, lane * L), c1 = min(a.NC, c0 + L);
+    double lw = 0.0, lp = 0.0;
+    for (int c = c0; c < c1; ++c) {
+      lw += s[2 * c];
+      lp += s[2 * c + 1];
     }
-    const int sel = tw > 0.0 ? 0 : 1;  // an empty residual draws from P itself
-    const double total = sel ? tp : tw;
-    const double t = (double)a.u_samp[b] * total;
-    double cum = 0.0;
-    int pick = -1, lastpos = -1;
-    for (int c = 0; c < a.NC; ++c) {
-      const double v = s[2 * c + sel];
-      if (v > 0.0) lastpos = c;
-      if (pick < 0 && cum + v > t) {
-        pick = c;
-        break;
+    double tw = lw, tp = lp;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const double ow = __shfl_up(tw, off, kWave), op = __shfl_up(tp, off, kWave);
+      tw += lane >= off ? ow : 0.0;
+      tp += lane >= off ? op : 0.0;
+    }
+    const int sel = __shfl(tw, kWave - 1, kWave) > 0.0 ? 0 : 1;  // an empty residual draws from P itself
+    const double own = sel ? lp : lw, inc = sel ? tp : tw;
+    const double t = (double)a.u_samp[b] * __shfl(inc, kWave - 1, kWave);
+    const uint64_t hit = __ballot(inc > t), some = __ballot(own > 0.0);
+    // the first lane whose chunks carry the cumulative weight past t, else the last with any weight
+    const int src = hit ? __builtin_ctzll(hit) : some ? 63 - __builtin_clzll(some) : 0;
+    const double before = src > 0 ? __shfl(inc, src - 1, kWave) : 0.0;
+    if (lane == src) {
+      double cum = before;
+      int pick = -1, lastpos = c0;
+      for (int c = c0; c < c1; ++c) {
+        const double v = s[2 * c + sel];
+        if (v > 0.0) lastpos = c;
+        if (hit && cum + v > t) {
+          pick = c;
+          break;
+        }
+        cum += v;
       }
-      cum += v;
+      if (hit && pick < 0) {  // the lane's own sum rounds below the scan's: its last weighted chunk
+        pick = lastpos;
+        cum -= s[2 * pick + sel];
+      }
+      s_last = !hit;
+      s_chunk = hit ? pick : lastpos;
+      s_t = t - cum;
+      s_sel = sel;
     }
-    s_last = pick < 0;
-    s_chunk = pick < 0 ? max(lastpos, 0) : pick;
-    s_t = t - cum;
-    s_tok = INT_MAX;
-    s_sel = sel;
+    if (lane == 0) s_tok = INT_MAX;
   }
   __syncthreads();
   const int c = s_chunk, sel = s_sel;
@@ -1434,6 +1492,7 @@ __global__ __launch_bounds__(kRT) void resid_pick_kernel(AcceptArgs a) {
   const int lo = c * a.chunk, hi = min(a.V, lo + a.chunk), len = hi - lo;
   // stage the chunk's weights in LDS with coalesced loads, then scan contiguous runs per thread
   const RowW rw = row_weights(a, b, r);
+#pragma unroll 4
   for (int j = tid; j < len; j += kRT) {
     float wt, pp;
     rw.at(lo + j, &wt, &pp);
@@ -1641,10 +1700,13 @@ __global__ __launch_bounds__(256) void probs_kernel(const float* logits, int64_t
     o[ix] = (y > -INFINITY && y >= t) ? __expf(y - mm) * inv : 0.f;
   }
 }
+// 16-byte accesses at any element's address: the hardware takes them, and a row of an odd vocabulary starts anywhere
+typedef u32x4 __attribute__((aligned(4))) u32x4_el4;
+typedef u32x4 __attribute__((aligned(2))) u32x4_el2;
+
 // Row-mapped form: out row out_rows[b K + j] of sequence b = P of logits row in_rows[b K + j] (whose
 // statistics are at [b, in_rows[..]]). An index outside its range skips the row: the maps are device
-// data the host cannot check. Four elements per thread per step (16-byte loads and stores) when vec.
-template <bool kVec>
+// data the host cannot check. Four elements per thread per step, the last V % 4 one per thread.
 __global__ __launch_bounds__(256) void probs_rows_kernel(const float* logits, int64_t bs, int64_t rs, int R, int V,
                                                          double rt, int ban, const float* m, const float* thr,
                                                          const double* zk, const int64_t* in_rows,
@@ -1663,25 +1725,21 @@ __global__ __launch_bounds__(256) void probs_rows_kernel(const float* logits, in
     const float y = make_y<true>(x, ix, rt, ban);
     return (y > -INFINITY && y >= t) ? __expf(y - mm) * inv : 0.f;
   };
-  if (kVec) {
-    const int n4 = V >> 2;
-    for (int j = blockIdx.x * 256 + threadIdx.x; j < n4; j += gridDim.x * 256) {
-      const u32x4 w = reinterpret_cast<const u32x4*>(row)[j];
-      float4 y;
-      y.x = p_of(__uint_as_float(w.x), 4 * j);
-      y.y = p_of(__uint_as_float(w.y), 4 * j + 1);
-      y.z = p_of(__uint_as_float(w.z), 4 * j + 2);
-      y.w = p_of(__uint_as_float(w.w), 4 * j + 3);
-      reinterpret_cast<float4*>(dst)[j] = y;
-    }
-  } else {
-    for (int ix = blockIdx.x * 256 + threadIdx.x; ix < V; ix += gridDim.x * 256) dst[ix] = p_of(row[ix], ix);
+  const int n4 = V >> 2;
+  for (int j = blockIdx.x * 256 + threadIdx.x; j < n4; j += gridDim.x * 256) {
+    const u32x4 w = reinterpret_cast<const u32x4_el4*>(row)[j];
+    u32x4 y;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] = __float_as_uint(p_of(__uint_as_float(w[e]), 4 * j + e));
+    reinterpret_cast<u32x4_el4*>(dst)[j] = y;
   }
+  const int ix = 4 * n4 + (int)threadIdx.x;
+  if (blockIdx.x == 0 && ix < V) dst[ix] = p_of(row[ix], ix);
 }
 
 // dst[b, k, :] = fp32(src[b, rows[b, k], :]) for bf16 (kBf16) or fp32 sources; a row index outside
-// [0, R) skips the row. 16-byte loads and stores when vec (8 bf16 or 4 fp32 elements a load).
-template <bool kBf16, bool kVec>
+// [0, R) skips the row. 16-byte loads (8 bf16 or 4 fp32 elements), the last V % 8 / V % 4 one per thread.
+template <bool kBf16>
 __global__ __launch_bounds__(256) void gather_rows_kernel(const void* src, int64_t sbs, int64_t srs, int R, int V,
                                                           const int64_t* rows, int K, float* dst, int64_t dbs,
                                                           int64_t drs) {
@@ -1691,34 +1749,29 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const void* src, int64
   if (i < 0 || i >= R) return;  // block-uniform
   float* d = dst + (int64_t)b * dbs + (int64_t)k * drs;
   const int64_t off = (int64_t)b * sbs + i * srs;
+  constexpr int E = kBf16 ? 8 : 4;
+  const int nv = V / E, ix = nv * E + (int)threadIdx.x;
   if (kBf16) {
     const uint16_t* s = static_cast<const uint16_t*>(src) + off;
-    if (kVec) {
-      for (int j = blockIdx.x * 256 + threadIdx.x; j < (V >> 3); j += gridDim.x * 256) {
-        const u32x4 w = reinterpret_cast<const u32x4*>(s)[j];
-        float4 lo, hi;
-        lo.x = __uint_as_float(w.x << 16);
-        lo.y = __uint_as_float(w.x & 0xffff0000u);
-        lo.z = __uint_as_float(w.y << 16);
-        lo.w = __uint_as_float(w.y & 0xffff0000u);
-        hi.x = __uint_as_float(w.z << 16);
-        hi.y = __uint_as_float(w.z & 0xffff0000u);
-        hi.z = __uint_as_float(w.w << 16);
-        hi.w = __uint_as_float(w.w & 0xffff0000u);
-        reinterpret_cast<float4*>(d)[2 * j] = lo;
-        reinterpret_cast<float4*>(d)[2 * j + 1] = hi;
+    for (int j = blockIdx.x * 256 + threadIdx.x; j < nv; j += gridDim.x * 256) {
+      const u32x4 w = reinterpret_cast<const u32x4_el2*>(s)[j];
+      u32x4 lo, hi;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        lo[2 * e] = w[e] << 16;
+        lo[2 * e + 1] = w[e] & 0xffff0000u;
+        hi[2 * e] = w[2 + e] << 16;
+        hi[2 * e + 1] = w[2 + e] & 0xffff0000u;
       }
-    } else {
-      for (int ix = blockIdx.x * 256 + threadIdx.x; ix < V; ix += gridDim.x * 256) d[ix] = bf2f(s[ix]);
+      reinterpret_cast<u32x4_el4*>(d)[2 * j] = lo;
+      reinterpret_cast<u32x4_el4*>(d)[2 * j + 1] = hi;
     }
+    if (blockIdx.x == 0 && ix < V) d[ix] = bf2f(s[ix]);
   } else {
     const float* s = static_cast<const float*>(src) + off;
-    if (kVec) {
-      for (int j = blockIdx.x * 256 + threadIdx.x; j < (V >> 2); j += gridDim.x * 256)
-        reinterpret_cast<float4*>(d)[j] = reinterpret_cast<const float4*>(s)[j];
-    } else {
-      for (int ix = blockIdx.x * 256 + threadIdx.x; ix < V; ix += gridDim.x * 256) d[ix] = s[ix];
-    }
+    for (int j = blockIdx.x * 256 + threadIdx.x; j < nv; j += gridDim.x * 256)
+      reinterpret_cast<u32x4_el4*>(d)[j] = reinterpret_cast<const u32x4_el4*>(s)[j];
+    if (blockIdx.x == 0 && ix < V) d[ix] = s[ix];
   }
 }
 }  // namespace
@@ -1738,19 +1791,10 @@ extern "C" int trida_truncated_probs_rows(const float* logits, int64_t B, int64_
                               out_batch_stride >= (Ro - 1) * out_row_stride + V)),
               TRIDA_ERR_ARG, "strides too small");
   if (K == 0) return TRIDA_OK;
-  const bool vec = V % 4 == 0 && row_stride % 4 == 0 && batch_stride % 4 == 0 && out_row_stride % 4 == 0 &&
-                   out_batch_stride % 4 == 0 && (((uintptr_t)logits | (uintptr_t)probs) & 15) == 0;
-  const int gx = (int)std::min<int64_t>(cdiv(V, 256 * (vec ? 4 : 1)), 256);
-  const dim3 grid(gx, (unsigned)(B * K));
-  const hipStream_t st = static_cast<hipStream_t>(stream);
-  if (vec)
-    hipLaunchKernelGGL((probs_rows_kernel<true>), grid, dim3(256), 0, st, logits, batch_stride, row_stride, (int)R,
-                       (int)V, 1.0 / (double)temperature, ban_of(ban_id, V), m, thr, zk, in_rows, out_rows, (int)K,
-                       (int)Ro, probs, out_batch_stride, out_row_stride);
-  else
-    hipLaunchKernelGGL((probs_rows_kernel<false>), grid, dim3(256), 0, st, logits, batch_stride, row_stride, (int)R,
-                       (int)V, 1.0 / (double)temperature, ban_of(ban_id, V), m, thr, zk, in_rows, out_rows, (int)K,
-                       (int)Ro, probs, out_batch_stride, out_row_stride);
+  const int gx = (int)std::min<int64_t>(cdiv(V, 256 * 4), 256);
+  hipLaunchKernelGGL(probs_rows_kernel, dim3(gx, (unsigned)(B * K)), dim3(256), 0, static_cast<hipStream_t>(stream), logits,
+                     batch_stride, row_stride, (int)R, (int)V, 1.0 / (double)temperature, ban_of(ban_id, V), m, thr, zk,
+                     in_rows, out_rows, (int)K, (int)Ro, probs, out_batch_stride, out_row_stride);
   return launch_status("probs_rows_kernel");
 }
 
@@ -1765,24 +1809,15 @@ extern "C" int trida_gather_rows(const void* src, int dtype, int64_t B, int64_t 
                               out_batch_stride >= (K - 1) * out_row_stride + V)),
               TRIDA_ERR_ARG, "strides too small");
   if (K == 0) return TRIDA_OK;
-  const int e = dtype == 1 ? 8 : 4;  // elements per 16-byte load
-  const bool vec = V % e == 0 && row_stride % e == 0 && batch_stride % e == 0 && out_row_stride % 4 == 0 &&
-                   out_batch_stride % 4 == 0 && (((uintptr_t)src | (uintptr_t)dst) & 15) == 0;
-  const int gx = (int)std::min<int64_t>(cdiv(V, 256 * (vec ? e : 1)), 256);
+  const int gx = (int)std::min<int64_t>(cdiv(V, 256 * (dtype == 1 ? 8 : 4)), 256);
   const dim3 grid(gx, (unsigned)(B * K));
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  if (dtype == 1 && vec)
-    hipLaunchKernelGGL((gather_rows_kernel<true, true>), grid, dim3(256), 0, st, src, batch_stride, row_stride, (int)R,
-                       (int)V, rows, (int)K, dst, out_batch_stride, out_row_stride);
-  else if (dtype == 1)
-    hipLaunchKernelGGL((gather_rows_kernel<true, false>), grid, dim3(256), 0, st, src, batch_stride, row_stride,
-                       (int)R, (int)V, rows, (int)K, dst, out_batch_stride, out_row_stride);
-  else if (vec)
-    hipLaunchKernelGGL((gather_rows_kernel<false, true>), grid, dim3(256), 0, st, src, batch_stride, row_stride,
-                       (int)R, (int)V, rows, (int)K, dst, out_batch_stride, out_row_stride);
+  if (dtype == 1)
+    hipLaunchKernelGGL((gather_rows_kernel<true>), grid, dim3(256), 0, st, src, batch_stride, row_stride, (int)R, (int)V,
+                       rows, (int)K, dst, out_batch_stride, out_row_stride);
   else
-    hipLaunchKernelGGL((gather_rows_kernel<false, false>), grid, dim3(256), 0, st, src, batch_stride, row_stride,
-                       (int)R, (int)V, rows, (int)K, dst, out_batch_stride, out_row_stride);
+    hipLaunchKernelGGL((gather_rows_kernel<false>), grid, dim3(256), 0, st, src, batch_stride, row_stride, (int)R, (int)V,
+                       rows, (int)K, dst, out_batch_stride, out_row_stride);
   return launch_status("gather_rows_kernel");
 }
 

@@ -13,10 +13,10 @@
 //       the sample-relative exponentials) take an exact radix select over the order-preserving keys of
 //       y, 8 bits per pass.
 //       Bound by the instructions of 16 waves per CU beside the row's bytes (two rows per CU at a time). 512
-//       rows of 248320, half of them peaked: 290 -> 189 us at T = 0.7, top_p = 0.95 (478 -> 123 at 0.5 / 0.8,
-//       259 -> 269 at 1.2 / 0.98, where two thirds of a row are kept and the boundary moves with each late
-//       token), 230 -> 122 with top_k = 50, 118 -> 96 (5.3 TB/s) untruncated; rows of 248319, which scalar loads
-//       served: 588 -> 181.
+//       rows of 248320, half of them peaked: 290 -> 184 us at T = 0.7, top_p = 0.95 (478 -> 122 at 0.5 / 0.8,
+//       259 -> 242 at 1.2 / 0.98, where two thirds of a row are kept and the boundary moves with each late
+//       token), 230 -> 122 with top_k = 50, 118 -> 98 (5.2 TB/s) untruncated; rows of 248319, which scalar loads
+//       served: 588 -> 169.
 //   resid_sums (grid NC x B): every block re-derives its sequence's accepted length from the drafted
 //       tokens' ratios P_i(d_i) / q_i(d_i), then sums the correction weights max(0, P_a - q_a) (P_K
 //       when every draft is accepted) and P_a over its chunk of the vocabulary, in fp64.
@@ -37,11 +37,12 @@ constexpr int kT = 512;  // threads of the truncation block
 constexpr int kTW = kT / kWave;
 constexpr int kSample = 2048;
 constexpr int kCap = 12288;  // LDS collection capacity (values)
+constexpr int kWaveCap = kCap / kTW;
 constexpr int kSortCap = 8192;  // values sorted at a time (a power of two, <= kCap)
 constexpr int kTopCount = 1024;  // entries at the top of a row that are always collected
 constexpr int kU = 4;            // 16-byte loads in flight per thread
 constexpr int kTileV = kT * kU;  // vectors per tile of the streaming pass
-constexpr int kQueue = 320;      // a wave's queue: up to 63 waiting elements and 4 new ones per lane
+constexpr int kQueue = 384;      // a wave's queue: up to 127 waiting elements and 4 new ones per lane
 constexpr int kSub = 1024;       // sub-bins of the boundary bin
 constexpr int kBins = 256;  // digits of one radix pass
 constexpr int kMaxTopK = 4096;
@@ -97,8 +98,8 @@ constexpr unsigned long long kMassMask = (1ull << kCountShift) - 1ull;
 constexpr int kMaxPackedV = (1 << 18) - 1;
 
 struct Shared {
-  float coll[kCap];
-  float queue[kTW][kQueue];  // each wave's elements above the floor, waiting for 64 to fold at once
+  float coll[kCap];           // the streaming pass: kWaveCap slots per wave; afterwards packed at the front
+  float queue[kTW][kQueue];  // each wave's elements above the floor, waiting to be folded 128 at a time
   unsigned long long hist[kNB + 1];
   unsigned cnt[kBins];  // radix-select digits
   double mass[kBins];
@@ -107,7 +108,7 @@ struct Shared {
   int ipar[6];
   int wlo[kSeg], whi[kSeg];  // the window each segment collected (bins, inclusive)
   int top[kSeg];             // and the bins [0, top)
-  int nseg[kSeg];            // collection fill after each segment
+  int nseg[kSeg][kTW];       // each wave's collected values after each segment (past kWaveCap: some were dropped)
   double dpar[4];
   unsigned umax;
 };
@@ -550,32 +551,34 @@ __device__ __forceinline__ void radix_resolve(const RowView& rv, const TruncArgs
 }
 
 // Keeps the collected logits whose bin lies in [lo, hi] and that came from a segment in the bit set
-// `segs` (entry j came from segment s when nseg[s-1] <= j < nseg[s]), packed at the front of
+// `segs` (entry j of wave w came from segment s when nseg[s-1][w] <= j < nseg[s][w]), packed at the front of
 // sh.coll; returns how many.
-__device__ __forceinline__ int compact_bins(const BinMap& bm, int n, int lo, int hi, unsigned segs) {
-  constexpr int kPer = kCap / kT;
-  float v[kPer];
+__device__ __forceinline__ int compact_bins(const BinMap& bm, int lo, int hi, unsigned segs) {
+  constexpr int kPer = kWaveCap / kT;  // steps per wave's slots
+  static_assert(kWaveCap % kT == 0, "whole steps");
+  float v[kTW * kPer];
   unsigned kp = 0u;
   const bool all = segs == (1u << kSeg) - 1u;
 #pragma unroll
-  for (int u = 0; u < kPer; ++u) {
-    if (u * kT >= n) break;  // block-uniform
-    const int j = u * kT + (int)threadIdx.x;
-    v[u] = j < n ? sh.coll[j] : -INFINITY;
+  for (int u = 0; u < kTW * kPer; ++u) {
+    const int w = u / kPer, j = (u % kPer) * kT + (int)threadIdx.x, n = min(sh.nseg[kSeg - 1][w], kWaveCap);
+    v[u] = -INFINITY;
+    if ((u % kPer) * kT >= n) continue;  // block-uniform
+    v[u] = j < n ? sh.coll[w * kWaveCap + j] : -INFINITY;
     const int bin = (int)bm.bin(v[u]);
     bool keep = j < n && bin >= lo && bin <= hi;
     if (!all) {
       int s = 0;
-      while (s < kSeg - 1 && j >= sh.nseg[s]) ++s;
+      while (s < kSeg - 1 && j >= sh.nseg[s][w]) ++s;
       keep = keep && ((segs >> s) & 1u);
     }
     kp |= (unsigned)keep << u;
   }
   double tot = 0.0;
-  int w = (int)block_excl_scan((double)__popc(kp), &tot);  // every read of sh.coll precedes its barriers
+  int at = (int)block_excl_scan((double)__popc(kp), &tot);  // every read of sh.coll precedes its barriers
 #pragma unroll
-  for (int u = 0; u < kPer; ++u)
-    if ((kp >> u) & 1u) sh.coll[w++] = v[u];
+  for (int u = 0; u < kTW * kPer; ++u)
+    if ((kp >> u) & 1u) sh.coll[at++] = v[u];
   __syncthreads();
   return (int)tot;
 }
@@ -606,8 +609,8 @@ __device__ __forceinline__ float below_bin(const BinMap& bm, int b) {
 
 // Streams a segment of the row in the logits' own units: the division by the temperature is folded into
 // the bin / exponent maps, and the exact y = x / T is only formed for the few collected values.
-// kHist: elements above x_lo (which lies below the floor, below_bin) wait in their wave's queue; each full
-// wave of 64 goes to the histogram and, those with a bin in [wlo, whi] or below `top`, to the collection.
+// kHist: elements above x_lo (which lies below the floor, below_bin) wait in their wave's queue; each two
+// full waves of 64 go to the histogram and, those with a bin in [wlo, whi] or below `top`, to the collection.
 // The others only add their mass (relative to exp(mref), less the rounding of bm.eB) to `tail`: fp32 over a
 // tile's 16 elements of a thread, fp64 across tiles. Without the queue every wave would run the 30 instructions of the
 // histogram for each of its elements, as some lane always has one above the floor (the block issues 16 waves'
@@ -616,26 +619,42 @@ __device__ __forceinline__ float below_bin(const BinMap& bm, int b) {
 // Otherwise only the elements between x_lo and x_hi are looked at, and those of the bins [wlo, whi] collected.
 template <bool kHist>
 __device__ __forceinline__ void stream_segment(const RowView& rv, const TruncArgs& a, const BinMap& bm, int s, float x_lo,
-                                               float x_hi, int top, int wlo, int whi, float& mx, double& tail) {
+                                               float x_hi, int top, int wlo, int whi, float& mx, double& tail,
+                                               int& have) {
   const int tid = threadIdx.x, lane = tid % kWave;
   float* queue = sh.queue[tid / kWave];
   int fill = 0;  // wave-uniform
   const unsigned wspan = (unsigned)(whi - wlo);
-  // folds the n (<= 64) elements at the end of the queue
+  // folds the n (<= 128) elements at the end of the queue, two per lane. The collected values go to the wave's own
+  // slots (kHist; `have` of them so far, wave-uniform), or behind a counter that the block shares.
   auto fold = [&](int n) {
     fill -= n;
-    bool in = false;
-    float x = 0.f;
-    if (lane < n) {
-      x = queue[fill + lane];
-      const unsigned bin = bm.bin(x);
+    float x[2];
+    uint64_t in[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int j = h * kWave + lane;
+      x[h] = queue[fill + min(j, n - 1)];
+      const unsigned bin = bm.bin(x[h]);
+      bool keep = (unsigned)((int)bin - wlo) <= wspan;
       if (kHist) {
-        atomicAdd(&sh.hist[bin], bm.packed(x, bin));
-        in = (int)bin < top;
+        keep = keep || (int)bin < top;
+        if (j < n) atomicAdd(&sh.hist[bin], bm.packed(x[h], bin));
       }
-      in |= (unsigned)((int)bin - wlo) <= wspan;
+      in[h] = __ballot(keep && j < n);
     }
-    append(x, in);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const bool mine = (in[h] >> lane) & 1ull;
+      if (kHist) {
+        const int at = have + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(in[h] >> 32),
+                                                            __builtin_amdgcn_mbcnt_lo((uint32_t)in[h], 0u));
+        if (mine && at < kWaveCap) sh.coll[(tid / kWave) * kWaveCap + at] = x[h];
+        have += __popcll(in[h]);
+      } else {
+        append(x[h], mine);
+      }
+    }
   };
   auto push = [&](float x, bool hot) {
     const uint64_t bal = __ballot(hot);
@@ -688,7 +707,7 @@ __device__ __forceinline__ void stream_segment(const RowView& rv, const TruncArg
       }
 #pragma unroll
       for (int e = 0; e < 4; ++e) one(xv[e], cold);
-      while (fill >= kWave) fold(kWave);
+      while (fill >= 2 * kWave) fold(2 * kWave);
     }
     if (kHist) tail += (double)cold;
   }
@@ -698,7 +717,7 @@ __device__ __forceinline__ void stream_segment(const RowView& rv, const TruncArg
     one(ix < rv.V && ix != a.ban ? rv.row[ix] : -INFINITY, cold);
     if (kHist) tail += (double)cold;
   }
-  while (fill > 0) fold(min(fill, kWave));
+  while (fill > 0) fold(min(fill, 2 * kWave));
 }
 
 // ---------------------------------------------------------------- the histogram, read by one wave
@@ -1082,7 +1101,6 @@ __global__ __launch_bounds__(kT, 4) void truncate_kernel(TruncArgs a) {
         if (bin < (unsigned)kNB) atomicAdd(&sh.hist[bin], bm.packed(x, bin));
       }
     }
-    if (tid == 0) sh.n = 0;
     __syncthreads();
     // ---- the streaming pass, kSeg segments: max, histogram down to the floor, collection of a window placed
     // from the sample's histogram and again from the row's own after every segment. Run again without
@@ -1091,6 +1109,7 @@ __global__ __launch_bounds__(kT, 4) void truncate_kernel(TruncArgs a) {
     int seen = 0, counted = ns;
     double tail = 0.0;
     bool floors = true;
+    int have = 0;
     int s = collect ? -1 : 0;
     while (true) {
       if (s >= 0) {
@@ -1099,19 +1118,23 @@ __global__ __launch_bounds__(kT, 4) void truncate_kernel(TruncArgs a) {
           sh.whi[s] = min(w_hi, floor_bin - 1);
           sh.top[s] = min(w_top, floor_bin);
         }
-        stream_segment<true>(rv, a, bm, s, collect ? below_bin(bm, floor_bin) : INFINITY, 0.f, w_top, w_lo, w_hi, mx, tail);
+        stream_segment<true>(rv, a, bm, s, collect ? below_bin(bm, floor_bin) : INFINITY, 0.f, w_top, w_lo, w_hi, mx, tail,
+                             have);
         ++passes;
         seen += seg_size(rv, s);
         counted = seen;
         tail_partials(tail);
+        if (tid % kWave == 0) sh.nseg[s][tid / kWave] = have;
         __syncthreads();
-        if (tid == 0) sh.nseg[s] = sh.n;
       }
       const int next = s + 1 < kSeg ? seg_size(rv, s + 1) : 0;
       if (s == kSeg - 1) {
         if (tid < kWave) find_boundary(lb, use_k, a.top_p, a.top_k, tail_total() * bm.cold_scale);
       } else if (collect && next > 0 && tid < kWave) {
-        const float room = fmaxf(0.75f * kCap - (float)min(sh.n, kCap), 0.f);
+        int got = 0;
+        if (s >= 0)
+          for (int w = 0; w < kTW; ++w) got += sh.nseg[s][w];
+        const float room = fmaxf(0.75f * kCap - (float)got, 0.f);
         place_window(lb, use_k, a.top_p, a.top_k, (float)counted / (float)V, s < 0 ? 0.0 : tail_total() * bm.cold_scale,
                      (float)next / (float)counted, s < 0 ? 0.2f * kCap : room / (float)(kSeg - 1 - s), floor_bin);
       }
@@ -1130,7 +1153,7 @@ __global__ __launch_bounds__(kT, 4) void truncate_kernel(TruncArgs a) {
         s = -1;  // the last window stands for the first segment
         __syncthreads();
         for (int j = tid; j <= kNB; j += kT) sh.hist[j] = 0ull;
-        if (tid == 0) sh.n = 0;
+        have = 0;
       } else if (collect && next > 0) {
         w_lo = sh.ipar[0];
         w_hi = sh.ipar[1];
@@ -1178,18 +1201,22 @@ __global__ __launch_bounds__(kT, 4) void truncate_kernel(TruncArgs a) {
       // keep what the segments whose window held [c_lo, c_hi] collected (and that fit the
       // collection); stream the others again
       unsigned complete = 0u;
-      for (int s = 0; s < kSeg; ++s)
-        complete |= (unsigned)(((c_lo >= sh.wlo[s] && c_hi <= sh.whi[s]) || c_hi < sh.top[s]) && sh.nseg[s] <= kCap) << s;
-      int n2 = compact_bins(bm, min(sh.n, kCap), c_lo, c_hi, complete);
+      for (int s = 0; s < kSeg; ++s) {
+        int fill = 0;
+        for (int w = 0; w < kTW; ++w) fill = max(fill, sh.nseg[s][w]);
+        complete |= (unsigned)(((c_lo >= sh.wlo[s] && c_hi <= sh.whi[s]) || c_hi < sh.top[s]) && fill <= kWaveCap) << s;
+      }
+      int n2 = compact_bins(bm, c_lo, c_hi, complete);
       if (complete != (1u << kSeg) - 1u) {
         __syncthreads();
         if (tid == 0) sh.n = n2;
         __syncthreads();
         const float x_lo = below_bin(bm, c_hi + 1), x_hi = c_lo > 1 ? below_bin(bm, c_lo - 2) : INFINITY;
         double none = 0.0;
+        int unused = 0;
         for (int s = 0; s < kSeg; ++s) {
           if ((complete >> s) & 1u) continue;
-          stream_segment<false>(rv, a, bm, s, x_lo, x_hi, 0, c_lo, c_hi, mx, none);
+          stream_segment<false>(rv, a, bm, s, x_lo, x_hi, 0, c_lo, c_hi, mx, none, unused);
           ++passes;
         }
         __syncthreads();

@@ -2,20 +2,23 @@
 // into q / k / v, l2norm of q and k per head, and the gates g = -exp(A_log) softplus(a + dt_bias),
 // beta = sigmoid(b).
 //
-// Launch: small grids take a grid of (sequence, row) x channel slices of 128 pieces (the C = conv_dim
-// channels of a row spread over several CUs; at batch 1 a row per block would leave most of the GPU idle
-// while each block pulls its 4 source rows and the whole conv weight); grids of >= 512 rows, which fill
-// the GPU anyway, one 256-thread block per row with up to 4 passes over its pieces. A thread owns 8
-// consecutive channels (one 16-byte piece) per pass; the Dk/8 threads of a q or k head reduce its sum of
-// squares with a row-local reduction.
+// Launch: a thread owns 8 consecutive channels (one 16-byte piece); the Dk/8 threads of a q or k head reduce
+// its sum of squares with a row-local reduction. Small grids take a grid of (sequence, row) x channel slices of 128
+// pieces (the C = conv_dim channels of a row spread over several CUs). From 512 rows on, a block takes up to 16
+// consecutive rows of a sequence: its thread keeps the conv weights and the last Kc - 1 source rows in registers,
+// so a row is loaded once (and its chunk's Kc - 1 predecessors) instead of by each of the Kc rows that
+// read it, and the weights (48 KB at C = 6144, as much as the row's four source rows) once per chunk.
 // Rounding follows the CPU oracle: conv and SiLU in fp32, rounded to bf16, then l2norm in fp32 of the
 // rounded values, rounded to bf16 again.
+#include <algorithm>
+
 #include "common.h"
 
 namespace trida {
 namespace {
 
 constexpr int kMaxKc = 4;
+constexpr int kNT = 128;  // threads, i.e. pieces, per block
 
 template <int CTRL>
 __device__ __forceinline__ float dpp(float x) {
@@ -57,6 +60,7 @@ struct PrepArgs {
   const int32_t* cu_seqlens;   // [B + 1] packed ragged rows, or null (B x T rows)
   int T, C, Kc, Hk, Hv, Dk, Dv;
   int64_t x_sb, x_st, ab_sb, ab_st;
+  int rows, chunks;  // rows per block and blocks per sequence (of T rows)
 };
 
 // Rows of sequence b: [row0, row0 + n) of the packed arrays. Contiguous form: n = T, row0 = b T (x and
@@ -96,134 +100,140 @@ __device__ __forceinline__ float softplus(float x) { return x > 20.f ? x : log1p
 
 // IDX: the pool / packed forms (slot indices, cu_seqlens) may be in use; without it those pointers are ignored
 // (null) and the plain form compiles without their loads and branches.
-template <int GW, int KC, int NT, int PASSES, bool IDX>  // lanes per q/k head = Dk / 8; conv width; threads; passes
-__global__ __launch_bounds__(NT) void gdn_prep_kernel(PrepArgs a) {
+// MULTI: blocks of `a.rows` rows, four at a time: the next four rows' loads go out before the current ones are
+// convolved. Otherwise one row per block.
+// 4096 rows of 6144 channels: 48 -> 36 us; 8 x 1024 rows of 8192 137 -> 74; 64 x 33 rows with pre_out 31 -> 23.
+template <int GW, int KC, bool MULTI, bool IDX>  // lanes per q/k head = Dk / 8; conv width
+__global__ __launch_bounds__(kNT) void gdn_prep_kernel(PrepArgs a) {
+  constexpr int G = MULTI ? 4 : 1;  // rows per step
   const int32_t* cu_seqlens = IDX ? a.cu_seqlens : nullptr;
   const int32_t* win_idx = IDX ? a.win_idx : nullptr;
   const int32_t* pre_idx = IDX ? a.pre_idx : nullptr;
-  const int t = blockIdx.x % a.T;
-  const int b = blockIdx.x / a.T;
+  const int t0 = (int)(blockIdx.x % a.chunks) * (MULTI ? a.rows : 1);
+  const int b = blockIdx.x / a.chunks;
   const SeqRows sr = seq_rows(cu_seqlens, a.T, b);
-  if (t >= sr.n) return;  // past a packed sequence's rows (block-uniform)
+  if (t0 >= sr.n) return;  // past a packed sequence's rows (block-uniform)
   const int T = sr.n;
+  const int t1 = MULTI ? min(T, t0 + a.rows) : t0 + 1;  // the block's rows [t0, t1)
   const int tid = threadIdx.x;
   const int key_dim = a.Hk * a.Dk;
   const int pieces = a.C / 8;
-  const int pbase = blockIdx.y * NT * PASSES;  // the block's first piece: a multiple of GW
+  const int p0 = blockIdx.y * kNT, p = p0 + tid;  // the block's first piece: a multiple of GW
+  const bool live = p < pieces;                   // lanes past the last piece load it and store nothing
+  const int c = min(p, pieces - 1) * 8;
   // the sequence's source rows (packed: row r of x at r x_st) and its window row
   const uint16_t* xb = cu_seqlens ? a.x + sr.row0 * a.x_st : a.x + (int64_t)b * a.x_sb;
   const int64_t ab0 = cu_seqlens ? sr.row0 * a.ab_st : (int64_t)b * a.ab_sb;
   const int wrow = win_idx ? win_idx[b] : b;
   const int prow_b = pre_idx ? pre_idx[b] : b;  // pre_out slot
   const uint16_t* wb = a.window + (int64_t)wrow * (a.Kc - 1) * a.C;
-  const int64_t orow = sr.row0 + t;  // output row (q, k, v, g, beta)
+  auto src = [&](int tau) {  // source row tau; negative rows come from the window
+    return *reinterpret_cast<const u32x4*>(tau >= 0 ? xb + (int64_t)tau * a.x_st + c : wb + (int64_t)(KC - 1 + tau) * a.C + c);
+  };
 
-  // every load of the block first (one memory round trip): the gate inputs, then per pass the KC source rows
-  // of the thread's 8 channels, their conv weights (8 channels x KC taps, contiguous: KC 16-byte pieces) and
-  // bias. The loads are unconditional (the gate inputs of blocks that do not write the gates, the bias from
-  // the conv weights when there is none: in bounds, unused), so that no branch splits the round trip. Lanes
-  // past the last piece load it (clamped) and store nothing; passes past it are skipped (block-uniform)
+  // every load of the first step first (one memory round trip): the gate inputs, the source rows of the thread's 8
+  // channels, their conv weights (8 channels x KC taps, contiguous: KC 16-byte pieces) and bias. The loads
+  // are unconditional (the gate inputs of blocks that do not write the gates, the bias from the conv
+  // weights when there is none: in bounds, unused), so that no branch splits the round trip.
   const bool gates = blockIdx.y == 0;  // block-uniform
   const int hg = min(tid, a.Hv - 1);
-  const uint16_t ar = a.a_in[ab0 + (int64_t)t * a.ab_st + hg];
-  const uint16_t br = a.b_in[ab0 + (int64_t)t * a.ab_st + hg];
+  const uint16_t ar = a.a_in[ab0 + (int64_t)t0 * a.ab_st + hg];
+  const uint16_t br = a.b_in[ab0 + (int64_t)t0 * a.ab_st + hg];
   const float alog = a.A_log[hg], dtb = a.dt_bias[hg];
   const uint16_t* cbias = a.conv_bias ? a.conv_bias : a.conv_w;
-  u32x4 xs[PASSES][KC], wsv[PASSES][KC], bsv[PASSES];
+  u32x4 xs[KC - 1 + G], wsv[KC];
 #pragma unroll
-  for (int ps = 0; ps < PASSES; ++ps) {
-    if (pbase + ps * NT >= pieces) break;
-    const int c = min(pbase + ps * NT + tid, pieces - 1) * 8;
+  for (int j = 0; j < KC - 1 + G; ++j) xs[j] = src(min(t0 - (KC - 1) + j, t1 - 1));
+#pragma unroll
+  for (int j = 0; j < KC; ++j) wsv[j] = reinterpret_cast<const u32x4*>(a.conv_w + (int64_t)c * KC)[j];
+  const u32x4 bsv = *reinterpret_cast<const u32x4*>(cbias + c);
+  float w[8][KC], bias[8];
+#pragma unroll
+  for (int ch = 0; ch < 8; ++ch)
 #pragma unroll
     for (int j = 0; j < KC; ++j) {
-      const int tau = t - (KC - 1) + j;  // source row; negative rows come from the window
-      const uint16_t* src = tau >= 0 ? xb + (int64_t)tau * a.x_st + c : wb + (int64_t)(KC - 1 + tau) * a.C + c;
-      xs[ps][j] = *reinterpret_cast<const u32x4*>(src);
-      wsv[ps][j] = reinterpret_cast<const u32x4*>(a.conv_w + (int64_t)c * KC)[j];
+      const int e = ch * KC + j;  // element of the 8 x KC weight block
+      const uint32_t word = wsv[e / 8][(e % 8) / 2];
+      w[ch][j] = __uint_as_float((e & 1) ? (word & 0xffff0000u) : (word << 16));
     }
-    bsv[ps] = *reinterpret_cast<const u32x4*>(cbias + c);
-  }
-  float av = bf2f(ar), bv = bf2f(br);
+  unpack8(bsv, bias);
+#pragma unroll
+  for (int ch = 0; ch < 8; ++ch) bias[ch] = a.conv_bias ? bias[ch] : 0.f;
 
+  for (int t = t0; t < t1; t += G) {
+    u32x4 xn[G];
+    if (MULTI && t + G < t1) {
 #pragma unroll
-  for (int ps = 0; ps < PASSES; ++ps) {
-    const int p0 = pbase + ps * NT;
-    if (p0 >= pieces) break;  // uniform
-    const int p = p0 + tid;
-    const bool live = p < pieces;
-    const int c = min(p, pieces - 1) * 8;
-    // the pre-conv rows a rollback rebuilds the window from: the block's own row is its last source row
-    if (a.pre_out && live) {
-      const int64_t prow = (int64_t)prow_b * a.T + t;
-      *reinterpret_cast<u32x4*>(a.pre_out + prow * a.C + c) = xs[ps][KC - 1];
+      for (int i = 0; i < G; ++i) xn[i] = src(min(t + G + i, t1 - 1));
     }
-    float acc[8];
-    {
-      float w[8][KC];
 #pragma unroll
-      for (int ch = 0; ch < 8; ++ch)
+    for (int i = 0; i < G; ++i) {
+      if (i > 0 && t + i >= t1) break;  // block-uniform
+      // the pre-conv rows a rollback rebuilds the window from: the row itself is its last source row
+      if (a.pre_out && live)
+        *reinterpret_cast<u32x4*>(a.pre_out + ((int64_t)prow_b * a.T + t + i) * a.C + c) = xs[i + KC - 1];
+      float acc[8];
 #pragma unroll
-        for (int j = 0; j < KC; ++j) {
-          const int e = ch * KC + j;  // element of the 8 x KC weight block
-          const uint32_t word = wsv[ps][e / 8][(e % 8) / 2];
-          w[ch][j] = __uint_as_float((e & 1) ? (word & 0xffff0000u) : (word << 16));
-        }
-      float bias[8];
-      unpack8(bsv[ps], bias);
-#pragma unroll
-      for (int ch = 0; ch < 8; ++ch) acc[ch] = a.conv_bias ? bias[ch] : 0.f;
+      for (int ch = 0; ch < 8; ++ch) acc[ch] = bias[ch];
 #pragma unroll
       for (int j = 0; j < KC; ++j) {
         float f[8];
-        unpack8(xs[ps][j], f);
+        unpack8(xs[i + j], f);
 #pragma unroll
         for (int ch = 0; ch < 8; ++ch) acc[ch] = fmaf(w[ch][j], f[ch], acc[ch]);
       }
 #pragma unroll
       for (int ch = 0; ch < 8; ++ch) acc[ch] = bf2f(f2bf(silu(acc[ch])));
-    }
-    // the q/k pieces come first (2 * key_dim / 8 of them, a multiple of GW) and are all live, so every
-    // group of GW lanes belongs to one head
-    if (p0 < 2 * key_dim / 8) {  // block-uniform: per-head l2norm (all lanes take part in the reduction)
-      const bool is_qk = c < 2 * key_dim;  // uniform across a GW-lane group
-      float ss = 0.f;
+      // the q/k pieces come first (2 * key_dim / 8 of them, a multiple of GW) and are all live, so every
+      // group of GW lanes belongs to one head
+      if (p0 < 2 * key_dim / 8) {  // block-uniform: per-head l2norm (all lanes take part in the reduction)
+        const bool is_qk = c < 2 * key_dim;  // uniform across a GW-lane group
+        float ss = 0.f;
 #pragma unroll
-      for (int ch = 0; ch < 8; ++ch) ss = fmaf(acc[ch], acc[ch], ss);
-      ss = lane_group_sum<GW>(ss);
-      if (is_qk) {
-        const float inv = rsqrtf(ss + 1e-6f);
+        for (int ch = 0; ch < 8; ++ch) ss = fmaf(acc[ch], acc[ch], ss);
+        ss = lane_group_sum<GW>(ss);
+        if (is_qk) {
+          const float inv = rsqrtf(ss + 1e-6f);
 #pragma unroll
-        for (int ch = 0; ch < 8; ++ch) acc[ch] *= inv;
+          for (int ch = 0; ch < 8; ++ch) acc[ch] *= inv;
+        }
+      }
+      if (live) {
+        const u32x4 o = pack8(acc);
+        const int64_t row = sr.row0 + t + i;  // output row (q, k, v, g, beta)
+        if (c < key_dim)
+          *reinterpret_cast<u32x4*>(a.q + row * key_dim + c) = o;
+        else if (c < 2 * key_dim)
+          *reinterpret_cast<u32x4*>(a.k + row * key_dim + (c - key_dim)) = o;
+        else
+          *reinterpret_cast<u32x4*>(a.v + row * (int64_t)a.Hv * a.Dv + (c - 2 * key_dim)) = o;
       }
     }
-    if (live) {
-      const u32x4 w = pack8(acc);
-      const int64_t row = orow;
-      if (c < key_dim)
-        *reinterpret_cast<u32x4*>(a.q + row * key_dim + c) = w;
-      else if (c < 2 * key_dim)
-        *reinterpret_cast<u32x4*>(a.k + row * key_dim + (c - key_dim)) = w;
-      else
-        *reinterpret_cast<u32x4*>(a.v + row * (int64_t)a.Hv * a.Dv + (c - 2 * key_dim)) = w;
-    }
-    // the new conv window (last Kc-1 rows of [window ++ x]): the last row's blocks, each its own pieces
-    if (a.window_out && t == T - 1 && live) {
-      for (int wr = 0; wr < a.Kc - 1; ++wr) {
-        const int tau = T - (a.Kc - 1) + wr;
-        const uint16_t* src = tau >= 0 ? xb + (int64_t)tau * a.x_st + c : wb + (int64_t)(a.Kc - 1 + tau) * a.C + c;
-        *reinterpret_cast<u32x4*>(a.window_out + ((int64_t)wrow * (a.Kc - 1) + wr) * a.C + c) =
-            *reinterpret_cast<const u32x4*>(src);
-      }
+    if (MULTI) {
+#pragma unroll
+      for (int j = 0; j < KC - 1; ++j) xs[j] = xs[j + G];
+#pragma unroll
+      for (int i = 0; i < G; ++i) xs[KC - 1 + i] = xn[i];
     }
   }
+  // the new conv window (last Kc-1 rows of [window ++ x]): the last row's blocks, each its own pieces
+  if (a.window_out && t1 == T && live) {
+    for (int wr = 0; wr < a.Kc - 1; ++wr)
+      *reinterpret_cast<u32x4*>(a.window_out + ((int64_t)wrow * (a.Kc - 1) + wr) * a.C + c) = src(T - (a.Kc - 1) + wr);
+  }
   if (gates) {
-    for (int hh = tid; hh < a.Hv; hh += NT) {
-      if (hh != tid) {  // more heads than threads: the later ones load their own inputs
-        av = bf2f(a.a_in[ab0 + (int64_t)t * a.ab_st + hh]);
-        bv = bf2f(a.b_in[ab0 + (int64_t)t * a.ab_st + hh]);
+    for (int i = tid; i < (t1 - t0) * a.Hv; i += kNT) {
+      const int t = t0 + i / a.Hv, hh = i % a.Hv;
+      float av = bf2f(ar), bv = bf2f(br), al = alog, dt = dtb;
+      if (i != tid || i != hg) {  // past the first row's heads: the inputs are loaded here
+        const int64_t at = ab0 + (int64_t)t * a.ab_st + hh;
+        av = bf2f(a.a_in[at]);
+        bv = bf2f(a.b_in[at]);
+        al = a.A_log[hh];
+        dt = a.dt_bias[hh];
       }
-      const int64_t o = orow * a.Hv + hh;
-      a.g[o] = -__expf(hh == tid ? alog : a.A_log[hh]) * softplus(av + (hh == tid ? dtb : a.dt_bias[hh]));
+      const int64_t o = (sr.row0 + t) * a.Hv + hh;
+      a.g[o] = -__expf(al) * softplus(av + dt);
       a.beta[o] = 1.f / (1.f + __expf(-bv));
     }
   }
@@ -262,42 +272,31 @@ extern "C" int trida_gdn_prep(const uint16_t* x, const uint16_t* window, const u
   TRIDA_CHECK(B * T < INT32_MAX, TRIDA_ERR_ARG, "gdn_prep: too many rows");
   PrepArgs a{x, window, conv_w, a_in, b_in, A_log, dt_bias, q, k, v, g, beta, window_out, pre_out,
              conv_bias, win_idx, pre_idx, cu_seqlens,
-             (int)T, (int)C, (int)Kc, (int)Hk, (int)Hv, (int)Dk, (int)Dv, x_sb, x_st, ab_sb, ab_st};
+             (int)T, (int)C, (int)Kc, (int)Hk, (int)Hv, (int)Dk, (int)Dv, x_sb, x_st, ab_sb, ab_st, 1, (int)T};
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // small grids: 128-piece slices, one per block; grids of >= 512 rows (which fill the GPU anyway): one
-  // block of 256 threads per row, up to 4 passes over its pieces, every pass's loads in flight together.
-  // The passes are a template argument: each holds its loads in registers (4 x 16-byte source pieces,
-  // 4 of weights, 1 of bias per thread), so a kernel built for more passes than the row needs would hold
-  // registers for nothing and fit fewer blocks per CU
-  const bool wide = B * T >= 512;
-  TRIDA_CHECK(!wide || C <= 8 * 256 * 4, TRIDA_ERR_ARG, "gdn_prep: conv_dim %lld above %d", (long long)C, 8 * 256 * 4);
-  const dim3 grid((unsigned)(B * T), wide ? 1u : (unsigned)cdiv(C / 8, 128));
+  // From 512 rows on a block takes several rows: as many as leave about 1536 blocks (12 waves per CU in flight), 4 to
+  // 16, in chunks of equal length: 9.6 -> 7.6 us at 512 rows (4 per block), 12.2 -> 8.3 at 16 x 33 with pre_out. 300
+  // rows take 5.3 us one per block, their launch and one memory round trip.
+  const bool multi = B * T >= 512;
+  TRIDA_CHECK(!multi || C <= 8 * 256 * 4, TRIDA_ERR_ARG, "gdn_prep: conv_dim %lld above %d", (long long)C, 8 * 256 * 4);
+  const int64_t slices = cdiv(C / 8, kNT);
+  const int64_t most = multi ? std::max<int64_t>(4, std::min<int64_t>(16, B * T * slices / 1536)) : 1;
+  a.chunks = (int)cdiv(T, most);
+  a.rows = (int)cdiv(T, a.chunks);
+  TRIDA_CHECK(B * a.chunks < INT32_MAX, TRIDA_ERR_ARG, "gdn_prep: too many rows");
+  const dim3 grid((unsigned)(B * a.chunks), (unsigned)slices);
   const bool idx = cu_seqlens || win_idx || pre_idx;
-#define TRIDA_PREP_KC2(GW, NT, PS, IX)                                                                     \
-  switch (Kc) {                                                                                            \
-    case 2: hipLaunchKernelGGL((gdn_prep_kernel<GW, 2, NT, PS, IX>), grid, dim3(NT), 0, st, a); break;     \
-    case 3: hipLaunchKernelGGL((gdn_prep_kernel<GW, 3, NT, PS, IX>), grid, dim3(NT), 0, st, a); break;     \
-    default: hipLaunchKernelGGL((gdn_prep_kernel<GW, 4, NT, PS, IX>), grid, dim3(NT), 0, st, a); break;    \
+#define TRIDA_PREP_KC(GW, MU, IX)                                                                        \
+  switch (Kc) {                                                                                          \
+    case 2: hipLaunchKernelGGL((gdn_prep_kernel<GW, 2, MU, IX>), grid, dim3(kNT), 0, st, a); break;      \
+    case 3: hipLaunchKernelGGL((gdn_prep_kernel<GW, 3, MU, IX>), grid, dim3(kNT), 0, st, a); break;      \
+    default: hipLaunchKernelGGL((gdn_prep_kernel<GW, 4, MU, IX>), grid, dim3(kNT), 0, st, a); break;     \
   }
-#define TRIDA_PREP_KC(GW, NT, PS)        \
-  if (idx) {                             \
-    TRIDA_PREP_KC2(GW, NT, PS, true)     \
-  } else {                               \
-    TRIDA_PREP_KC2(GW, NT, PS, false)    \
-  }
-  const int64_t passes = wide ? cdiv(C / 8, 256) : 1;
-#define TRIDA_PREP_LAUNCH(GW)          \
-  if (!wide) {                         \
-    TRIDA_PREP_KC(GW, 128, 1)          \
-  } else if (passes <= 1) {            \
-    TRIDA_PREP_KC(GW, 256, 1)          \
-  } else if (passes == 2) {            \
-    TRIDA_PREP_KC(GW, 256, 2)          \
-  } else if (passes == 3) {            \
-    TRIDA_PREP_KC(GW, 256, 3)          \
-  } else {                             \
-    TRIDA_PREP_KC(GW, 256, 4)          \
-  }
+#define TRIDA_PREP_LAUNCH(GW)                        \
+  if (multi && idx) { TRIDA_PREP_KC(GW, true, true) }     \
+  else if (multi) { TRIDA_PREP_KC(GW, true, false) }      \
+  else if (idx) { TRIDA_PREP_KC(GW, false, true) }        \
+  else { TRIDA_PREP_KC(GW, false, false) }
   switch (Dk) {
     case 32: TRIDA_PREP_LAUNCH(4) break;
     case 64: TRIDA_PREP_LAUNCH(8) break;
@@ -305,6 +304,5 @@ extern "C" int trida_gdn_prep(const uint16_t* x, const uint16_t* window, const u
   }
 #undef TRIDA_PREP_LAUNCH
 #undef TRIDA_PREP_KC
-#undef TRIDA_PREP_KC2
   return launch_status("gdn_prep");
 }

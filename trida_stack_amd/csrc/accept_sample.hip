@@ -82,7 +82,7 @@ __device__ __forceinline__ int next_pow2(int n) {
 }
 
 // Value histogram of the streaming pass: 2048 bins of 1/32 nat over d = y - mref in (-24, 40]
-// (mref = the sample max); bin 0 holds the largest values. Bin kNB is the spare bin: entries with d > 40, which are
+// (mref = the sample max, rounded to a bin); bin 0 holds the largest values. Bin kNB is the spare bin: entries with d > 40, which are
 // caught afterwards from the row max and send the row to the radix select, and a few at the lower end. The
 // others with d <= -24, -inf entries, the banned id and padding lanes only add their mass to the total.
 // Each bin is one 64-bit LDS word: the count in bits 46..63 and, below, the sum of r * 2^26 with
@@ -298,21 +298,23 @@ __device__ __forceinline__ double bin_mass(unsigned long long h, double scale) {
 
 struct BinMap {  // the per-row coefficients of the element -> bin / exponent maps
   float tA, tB;       // t = fma(x, tA, tB)
-  float rf, rl, nm;   // d = x (rf + rl) + nm = x / T - mref
+  float nm;           // -mref
+  double rt;          // 1 / T
   float eA, eB;       // exp(d) = exp2(fma(x, eA, eB)) * cold_scale
   double cold_scale;  // what the rounding of eB took away
   __device__ unsigned bin(float x) const { return bin_of_t(fmaf(x, tA, tB)); }
   // an element's histogram entry: a count of one and its mass relative to its bin's upper edge
   __device__ unsigned long long packed(float x, unsigned bin) const {
-    const float d = fmaf(x, rl, fmaf(x, rf, nm));
+    // y = x / T as the kept set and the probabilities round it (a likely token's y of 16..32 rounds by up to 1e-6,
+    // which would be an error of its mass); mref and the edge are multiples of 2^-5, so that d is exact
     const float edge = fmaf((float)bin, -1.f / kPerNat, kTop);
-    const float r = __builtin_amdgcn_exp2f((d - edge) * 1.44269504f) * 0x1p26f;
+    const float d = exact_y<true>(x, rt) + (nm - edge);
+    const float r = __builtin_amdgcn_exp2f(d * 1.44269504f) * 0x1p26f;
     return (1ull << kCountShift) | (unsigned long long)(unsigned)r;
   }
-  __device__ void set(double rt, float mref) {
-    rf = (float)rt;
-    rl = (float)(rt - (double)rf);
-    tA = -kPerNat * rf;
+  __device__ void set(double rt_, float mref) {
+    rt = rt_;
+    tA = -kPerNat * (float)rt;
     tB = kPerNat * (kTop + mref);
     nm = -mref;
     const double l2e = 1.4426950408889634;
@@ -1090,6 +1092,7 @@ __global__ __launch_bounds__(kT, 4) void truncate_kernel(TruncArgs a) {
     for (int j = tid; j <= kNB; j += kT) sh.hist[j] = 0ull;
     smax = block_max(smax);
     mref = smax > -INFINITY ? exact_y<kDiv>(smax, a.rt) : 0.f;
+    if (fabsf(mref) < 0x1p18f) mref = rintf(mref * kPerNat) / kPerNat;  // a whole bin: see BinMap::packed
     bm.set(a.rt, mref);
     LaneBins lb;
     if (tid < kWave) lb.init();

@@ -1,0 +1,65 @@
+"""GPU: canvas attention at the edges of its tiles: query rows around one and two row tiles per wave and the extra
+rows of a last tile, keys around a 64-key step, scales of either sign and zero, scores that keep rising (the
+running max moves at every step) and rows of very different magnitude in one tile; against the oracle."""
+import pytest
+import torch
+
+from oracle import attention as A
+from trida_stack_amd import kernels as K
+
+pytestmark = pytest.mark.gpu
+TOL = 2e-2  # normwise max-abs of bf16 products, as the other attention tests
+
+
+def rel(a, b):
+    a, b = a.float().cpu(), b.float().cpu()
+    return float((a - b).abs().max() / b.abs().max().clamp_min(1e-30))
+
+
+def check(gpu, B, T, Hq, Hkv, D, prefix, mode, scale=None, shape=lambda q, k, v: (q, k, v), splits=0):
+    g = torch.Generator().manual_seed(T * 7 + D + mode)
+    L = max(prefix) + T
+    q, k, v = shape(torch.randn(B, T, Hq, D, generator=g), torch.randn(B, Hkv, L, D, generator=g),
+                    torch.randn(B, Hkv, L, D, generator=g))
+    q, k, v = (t.to(torch.bfloat16) for t in (q, k, v))
+    # the oracle's scale is D^-0.5: the factor beyond it goes into its fp32 queries
+    f = 1.0 if scale is None else scale * D ** 0.5
+    ref = A.canvas_attention(q.float() * f, k.float(), v.float(), prefix, mode, T // 2)
+    kw = {} if scale is None else dict(scale=scale)
+    out = K.attn_canvas(q.to(gpu), k.to(gpu), v.to(gpu), torch.tensor(prefix, dtype=torch.int32, device=gpu), mask_mode=mode,
+                        n_clean=T // 2, splits=splits, **kw)
+    assert rel(out, ref) < TOL
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 63, 64, 65, 96, 127, 128, 129, 144, 145, 256, 260])
+def test_query_rows(gpu, D, rows):
+    check(gpu, 1, rows, 1, 1, D, [100], 0)
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("rows", [129, 144, 272])
+def test_extra_rows(gpu, D, rows):
+    B = 140  # more query tiles than CUs: the last one of <= 16 rows joins the tile before it
+    check(gpu, B, rows, 2, 2, D, [(13 * i) % 90 for i in range(B)], 2)
+
+
+@pytest.mark.parametrize("keys", [1, 63, 64, 65, 127, 128, 129, 193])
+@pytest.mark.parametrize("splits", [1, 2, 0])
+def test_key_steps(gpu, keys, splits):
+    check(gpu, 2, 1, 4, 2, 256, [keys - 1, max(keys - 2, 0)], 1, splits=splits)
+
+
+@pytest.mark.parametrize("scale", [0.0, -0.0625, 0.25])
+def test_scales(gpu, scale):
+    check(gpu, 1, 33, 8, 2, 128, [150], 0, scale=scale)
+
+
+@pytest.mark.parametrize("T", [4, 33])
+def test_rising_scores(gpu, T):
+    def shape(q, k, v):
+        ramp = torch.linspace(0.01, 3.0, k.shape[2])[None, None, :, None]
+        rows = torch.logspace(-2, 1, q.shape[1])[None, :, None, None]
+        return q.abs() * rows, k.abs() * ramp, v
+
+    check(gpu, 1, T, 4, 1, 256, [500], 0, shape=shape, splits=1)

@@ -30,6 +30,11 @@ HIPCC_FLAGS = [
     f"-I{PKG.parent / 'include'}",
 ]
 
+# attention.hip: MFMA accumulators in the ordinary registers. Its kernels of head dim 256 hold more than 256 registers,
+# for which the compiler would keep the accumulators in the accumulation half and move them at every rescale and
+# loop edge (about 400 moves a step, a third of its instructions).
+FILE_FLAGS = {"attention": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+
 
 def hipcc() -> str:
     for cand in (os.environ.get("HIPCC"), "/opt/rocm/bin/hipcc", shutil.which("hipcc")):
@@ -40,7 +45,7 @@ def hipcc() -> str:
 
 def _compile(src: Path) -> Path:
     obj = OBJ / (src.stem + ".o")
-    cmd = [hipcc(), *HIPCC_FLAGS, "-c", str(src), "-o", str(obj)]
+    cmd = [hipcc(), *HIPCC_FLAGS, *FILE_FLAGS.get(src.stem, []), "-c", str(src), "-o", str(obj)]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src.name}:\n{r.stdout}\n{r.stderr}")

@@ -7,16 +7,14 @@
 //   mask 1 (draft, bidirectional) always
 //   mask 2 (canvas, mixed)        j <= t for t < n_clean, always for t >= n_clean
 //
-// attn_partial: workgroup = (sequence, KV head, query tile of <= 128 rows, key split), 8 waves of 16
-//   rows each. Per 64-key step, K (XOR-swizzled) and V (row-major, padded rows) are staged in LDS while
-//   the next step is loaded into registers; every wave computes S^T = K Q^T for its rows with
-//   v_mfma_f32_16x16x32_bf16 (Q and K fragments from LDS), runs the online softmax within the wave, and
-//   accumulates O^T += V^T P^T with the V^T fragments read by ds_read_b64_tr_b16.
+// attn_partial: workgroup = (sequence, KV head, query tile of <= 128 rows, key split), 4 waves of 16 or 32
+//   rows each. Per 64-key step, K and V are staged in one of two LDS buffers (swizzled, loaded to LDS directly while
+//   the other is in use); every wave computes S^T = K Q^T for its rows with v_mfma_f32_16x16x32_bf16 (K fragments
+//   from LDS, Q in registers), runs the online softmax within the wave, and accumulates O^T += V^T P^T
+//   with the V^T fragments read by ds_read_b64_tr_b16.
 //   Writes the unnormalised O (bf16), row max and row sum (fp32) of its split. A last tile of <= 16
 //   rows can join the tile before it as its extra rows (a canvas of 33 rows x 4 heads = 128 + 4), so
-//   the keys stream once for all rows: wave w takes key tile w % 4 of every step for them (an online
-//   softmax of its own over those keys) and half w / 4 of their output columns, from the K / V
-//   fragments it reads for its own rows; the workgroup merges the four key-tile states at the end.
+//   the keys stream once for all rows.
 // attn_combine: merges the splits per row (log-sum-exp weights), applies the optional output gate
 //   sigmoid(gate) and writes bf16; attn_combine2 does the same for exactly two splits in one memory round
 //   trip per row.
@@ -30,13 +28,22 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kNW = 8;              // waves per workgroup
-constexpr int kWR = 16;             // query rows per wave (one MFMA row tile)
-constexpr int kMT = kNW * kWR;      // query rows per workgroup, before extra rows
+constexpr int kNW = 4;              // waves per workgroup
+constexpr int kWR = 16;             // an MFMA row tile
+constexpr int kMT = kNW * 2 * kWR;  // query rows per workgroup (two row tiles per wave), before extra rows
 constexpr int kMTX = kMT + kWR;     // with a last tile's <= 16 extra rows
 constexpr int kKB = 64;             // keys per step
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kMaxLptSeqs = 256;  // batches up to this size are scheduled longest-first
+
+// The max over the four lanes of a row (l, l ^ 16, l ^ 32, l ^ 48), without a trip through LDS: each swap leaves a
+// lane's value and its partner's in the two results
+__device__ __forceinline__ float row_max(float x) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
 
 template <int CTRL>
 __device__ __forceinline__ float dpp(float x) {
@@ -67,58 +74,96 @@ struct AttnArgs {
   int frag;
 };
 
-// LDS tiles of one 64-key step, 16-byte groups XOR-swizzled so that both the staging writes and the
-// MFMA fragment reads touch distinct bank groups:
-//   K [key][D]   group g of key k stored at g ^ (k & 7) (16-byte fragment reads, 8 keys per 8 lanes)
-//   V [key][D + 16] row-major, rows padded by 32 bytes: the V^T fragments of the P V^T product come from
-//                ds_read_b64_tr_b16 (8 bytes of one key per lane, handed out transposed), and the 32 lanes
-//                of a half-wave, 8 keys x 32 bytes, then fall on distinct banks; a fragment's address is
-//                linear in its column tile (immediate offsets)
+// LDS tiles of one 64-key step, [key][D] with the pieces of a key XOR-swizzled so that the MFMA fragment reads
+// touch distinct banks:
+//   K  16-byte group g of key k at g ^ (k & 7) (16-byte fragment reads, 8 keys per 8 lanes)
+//   V  32-byte unit u of key k at u ^ vswz(k): the V^T fragments of the P V^T product come from ds_read_b64_tr_b16
+//      (8 bytes of one key per lane, handed out transposed), and the 32 lanes of a half-wave, 8 keys x 32 bytes,
+//      then fall on distinct banks
+// The tiles are written by global_load_lds: a wave's load fills 1 KB in lane order, so the swizzle is in the
+// address that each lane loads from.
 template <int D>
 __device__ __forceinline__ int k_off(int key, int grp) { return key * D + ((grp ^ (key & 7)) << 3); }
-constexpr int kVPad = 16;
 template <int D>
-__device__ __forceinline__ int v_off(int key, int grp) { return key * (D + kVPad) + (grp << 3); }
+__device__ __forceinline__ int vswz(int key) { return D >= 128 ? key & 7 : (key >> 1) & 3; }
+template <int D>
+__device__ __forceinline__ int v_off(int key, int unit) { return key * D + ((unit ^ vswz<D>(key)) << 4); }
+
+// 64 lanes x 16 bytes from each lane's address to LDS at `lds` (bytes, wave-uniform) + 16 lane, asynchronously: counted by
+// vmcnt, no register written. In asm because the compiler would wait for it before every later LDS read.
+__device__ __forceinline__ void load_lds16(const uint16_t* src, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory", "m0");
+}
+__device__ __forceinline__ uint32_t lds_addr(const void* p) { return (uint32_t)(uintptr_t)p; }
+// Every wave's loads to LDS have arrived and its LDS reads have returned: the other tile buffer may be overwritten.
+__device__ __forceinline__ void step_barrier() {
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// Fragment reads at an LDS byte address: a lane's addresses within a tile differ by constants (instruction
+// offsets) from a few that depend on the swizzle, FragAt; left to the compiler, each of the step's fragments had
+// an address register of its own.
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
 // ds_read_b64_tr_b16 (gfx950): in each group of 16 lanes, lane 4 a + b receives element b of the 8-byte
 // reads of lanes a, a + 4, a + 8 and a + 12 (in that order). A lane of group g reading key key0 + 4 g +
 // (lane % 16) / 4 at columns d0 + 4 (lane % 4) .. + 3 thus receives V[key0 + 4 g + j][d0 + lane % 16] for
 // j = 0..3: four keys of its V^T row, in the k slots of the MFMA's A operand.
 template <int D>
-__device__ __forceinline__ s16x4 vt_frag4(const uint16_t* sV, int key0, int d0, int l) {
-  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-  const int key = key0 + 4 * (l / 16) + (l % 16) / 4, col = d0 + 4 * (l % 4);
-  const uint16_t* p = sV + v_off<D>(key, col / 8) + col % 8;
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uint32_t)(uintptr_t)p);
-}
+struct FragAt {
+  static constexpr int VU = D >= 128 ? 8 : 4;  // units of a key within the V swizzle's reach
+  uint32_t k[2], v[VU];
+  __device__ __forceinline__ FragAt(int l) {
+    const int key = 4 * (l / 16) + (l % 16) / 4;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) k[i] = 2 * k_off<D>(l % 16, 4 * i + l / 16);
+#pragma unroll
+    for (int u = 0; u < VU; ++u) v[u] = 2 * (v_off<D>(key, u) + 4 * (l % 4));
+  }
+  // K (or Q) row key0 + lane % 16, columns 32 kc + 8 (lane / 16) .. + 7; key0 a multiple of 16
+  __device__ __forceinline__ bf16x8 row(uint32_t tile, int key0, int kc) const {
+    return as_bf16x8(*(lds_u32x4*)(tile + k[kc % 2] + (uint32_t)(key0 * D * 2 + (kc / 2) * 128)));
+  }
+  // V^T row 16 ct + lane % 16, keys key0 + 4 (lane / 16) .. + 3
+  __device__ __forceinline__ s16x4 col(uint32_t tile, int key0, int ct) const {
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (lds_s16x4*)(tile + v[ct % VU] + (uint32_t)(key0 * D * 2 + (ct / VU) * (VU * 32))));
+  }
+};
 
-// Workgroup = (sequence, KV head, query tile of kMT rows, key split); 8 waves, wave w owns rows
-// [16 w, 16 w + 16) of the tile. Per 64-key step: K and V^T are staged in LDS (the next step's K / V
-// are loaded into registers meanwhile) and the wave forms the transposed products S^T = K Q^T and
-// O^T += V^T P^T on v_mfma_f32_16x16x32_bf16, so lane l holds 16 scores and 256 / 4 output values of
-// one query row (l % 16): the online softmax of a row is the lane's own, completed across its four
-// lane groups by two xor exchanges, and its probabilities are, as computed, the B operand of the
-// product with V (a 32-key block takes slots 8 g + j = keys 32 kk + 4 g + j and 32 kk + 16 + 4 g + j - 4,
-// which is where the two key tiles' accumulators put them). O is rescaled only when a row's running max
-// moved. Writes the unnormalised O, the row max (log2 domain) and the row sum of its split.
-// Extra rows (the last tile's kMT .. kMT + 15): wave w forms the 16 keys x 16 rows of key tile w % 4 of
-// their S^T with the K fragments of its own product (the extra rows' Q from LDS), runs an online softmax
-// over the keys it sees this way, and accumulates columns [D/2 (w / 4), D/2 (w / 4 + 1)) of their O^T on
-// v_mfma_f32_16x16x16_bf16, whose B operand is the S^T accumulator layout as it stands (A: 4 keys of a
-// V^T row from the staged tile). No barrier inside a step; after the last one the waves of each column
-// half merge their four key tiles' states through LDS in key-tile order.
-template <int D>
-__global__ __launch_bounds__(kNW* kWave) void attn_partial_kernel(AttnArgs a) {
+// Workgroup = (sequence, KV head, query tile of kMT rows, key split); 4 waves, wave w owns RT row tiles of 16: rows
+// [16 RT w, 16 RT (w + 1)) of the tile, their Q as B fragments in registers. Per 64-key step, K and V are staged
+// in one of two LDS buffers while the next step's tiles stream into the other (global_load_lds), and the
+// wave forms the transposed products S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_16x16x32_bf16, so lane l holds
+// 16 scores and 256 / 4 output values of one query row (l % 16) of each tile: the online softmax of a row is
+// the lane's own, completed across its four lane groups by two xor exchanges, and its probabilities are, as
+// computed, the B operand of the product with V (a 32-key block takes slots 8 g + j = keys 32 kk + 4 g + j
+// and 32 kk + 16 + 4 g + j - 4, which is where the two key tiles' accumulators put them). O is rescaled only
+// when a row's running max moved. Writes the unnormalised O, the row max (log2 domain) and the row sum of its split.
+// Each K and V fragment read feeds RT products: what bounds a step is LDS reads (each wave reads both tiles, 64
+// KB at D = 256), so 32 rows per wave halve them against 16. RT = 1 serves tiles of <= 64 rows, whose waves
+// would otherwise be idle.
+// Against 8 waves of 16 rows, tiles staged through registers between two barriers and Q in LDS: 64 sequences of 33
+// rows and 512-4096 keys 253 -> 215 us (head dim 256; 128: 134 -> 99), a 512-row chunk behind 3584 keys 82 -> 67,
+// 33 rows over 8192 keys 34 -> 31, 64 sequences of one row 117 -> 111 (5.4 TB/s of keys). A step of 32 rows per
+// wave takes about 3 us of MFMA, LDS reads and softmax one after the other, as 2 x 64 KB of tiles leave room for
+// one workgroup per CU.
+// Extra rows (EXTRA: the last tile's kMT .. kMT + 15): a third row tile of every wave, from the K fragments the wave
+// reads for its own rows (Q from LDS); of their O^T, wave w accumulates the column tiles [XC w, XC (w + 1)).
+template <int D, int RT, bool EXTRA>
+__global__ __launch_bounds__(kNW* kWave, D == 256 ? 1 : 2) void attn_partial_kernel(AttnArgs a) {
   constexpr int KC = D / 32;         // 32-wide k-chunks of the head dim (QK^T)
   constexpr int CT = D / 16;         // 16-column tiles of O
   constexpr int GPR = D / 8;         // 16-byte groups per K row
   constexpr int NT = kNW * kWave;
-  constexpr int NKG = kKB * GPR / NT;  // K groups staged per thread
-  constexpr int XH = CT / 2;  // O^T column tiles of the extra rows per wave (half of them)
-  __shared__ __align__(16) uint16_t sQ[kMT * D];  // [row][D], groups swizzled by row & 7 (as K)
-  __shared__ __align__(16) uint16_t sQx[kWR * D];  // the extra rows, the same layout
-  __shared__ __align__(16) uint16_t sK[kKB * D];
-  __shared__ __align__(16) uint16_t sV[kKB * (D + kVPad)];
-  __shared__ float sXm[kNW][kWR], sXl[kNW][kWR];  // the extra rows' per-wave running max and sum
+  constexpr int KPL = kWave / GPR;          // keys per wave load (1 KB)
+  constexpr int NL = kKB / (KPL * kNW);     // loads per wave of a tile
+  constexpr int ST = RT + (EXTRA ? 1 : 0);  // row tiles that form scores: the extra rows are the last one
+  constexpr int XC = CT / kNW;              // column tiles of the extra rows per wave
+  constexpr int TILE = kKB * D;
+  // [buffer][K, V] tiles
+  __shared__ __align__(16) uint16_t sKV[2][2][TILE];
+  __shared__ __align__(16) uint16_t sQx[EXTRA ? kWR * D : 8];  // the extra rows' Q, as K
 
   const int tid = threadIdx.x, w = tid / kWave, l = tid % kWave;
   const int per_pair = a.S * a.QT;                  // workgroups per (sequence, KV head)
@@ -189,81 +234,89 @@ __global__ __launch_bounds__(kNW* kWave) void attn_partial_kernel(AttnArgs a) {
   const uint16_t* kh = a.k_cache + ((int64_t)b * a.Hkv + hk) * a.Lmax * D;
   const uint16_t* vh = a.v_cache + ((int64_t)b * a.Hkv + hk) * a.Lmax * D;
 
-  // ---- prefetch registers: K and V groups (coalesced rows)
-  u32x4 kreg[NKG], vreg[NKG];
-  auto load_step = [&](int kb) {
-    const int key0 = kb * kKB;
+  // ---- the step's tiles, key KPL (w + 4 j) + l / GPR of each lane's load j (keys past the last one re-read it). The
+  // swizzles depend on the key's low bits only, the same for every j.
+  const int lkey = KPL * w + l / GPR, lg = l % GPR;
+  const uint16_t* ksrc = kh + ((lg ^ (lkey & 7)) << 3);
+  const uint16_t* vsrc = vh + ((((lg >> 1) ^ vswz<D>(lkey)) << 4) + ((lg & 1) << 3));
+  auto load_step = [&](int kb, int buf) {
 #pragma unroll
-    for (int j = 0; j < NKG; ++j) {
-      const int gi = tid + j * NT;
-      const int key = min(key0 + gi / GPR, nk - 1);
-      kreg[j] = *reinterpret_cast<const u32x4*>(kh + (int64_t)key * D + (gi % GPR) * 8);
-      vreg[j] = *reinterpret_cast<const u32x4*>(vh + (int64_t)key * D + (gi % GPR) * 8);
+    for (int j = 0; j < NL; ++j) {
+      const int64_t row = (int64_t)min(kb * kKB + lkey + j * KPL * kNW, nk - 1) * D;
+      const uint32_t at = lds_addr(&sKV[buf][0][0]) + (uint32_t)((w + j * kNW) * 1024);
+      load_lds16(ksrc + row, __builtin_amdgcn_readfirstlane(at));
+      load_lds16(vsrc + row, __builtin_amdgcn_readfirstlane(at + TILE * 2));
     }
   };
-  // the first step's K / V loads go out with the Q loads: one memory latency for both
-  load_step(kb0);
+  load_step(kb0, 0);
 
-  // ---- the tile's Q rows into LDS (padding rows zero); read back as A fragments every step. Every
-  // load of the tile is issued before the first store, so the staging costs one memory latency.
+  // ---- the Q rows as B fragments (rows past the tile zero)
+  const int wr0 = w * RT * kWR;  // the wave's first row
+  bf16x8 qf[RT][KC];
   {
-    constexpr int QPT = kMT * GPR / NT;  // 16-byte pieces per thread
-    static_assert(kWR * GPR <= NT, "one piece of the extra rows per thread");
-    u32x4 qv[QPT], qx = u32x4{0u, 0u, 0u, 0u};
-    auto q_at = [&](int m, int grp) {
+    auto q_at = [&](int m, int kc) {
       const int t = m / a.G, g = m % a.G;
-      return *reinterpret_cast<const u32x4*>(a.q + (((int64_t)b * a.T + t) * a.Hq + hk * a.G + g) * D + grp * 8);
+      return as_bf16x8(*reinterpret_cast<const u32x4*>(a.q + (((int64_t)b * a.T + t) * a.Hq + hk * a.G + g) * D + kc * 32 +
+                                                       (l / 16) * 8));
     };
+    const bf16x8 zero = as_bf16x8(u32x4{0u, 0u, 0u, 0u});
+    // the softmax takes a scale >= 0: a negative one's sign goes to Q
+    auto neg = [](bf16x8 v) { return as_bf16x8(__builtin_bit_cast(u32x4, v) ^ 0x80008000u); };
 #pragma unroll
-    for (int j = 0; j < QPT; ++j) {
-      const int gi = tid + j * NT;
-      qv[j] = q_at(m0 + min(gi / GPR, rows - 1), gi % GPR);
-    }
-    if (nx > 0 && tid < kWR * GPR) qx = q_at(m0 + kMT + min(tid / GPR, nx - 1), tid % GPR);
+    for (int rt = 0; rt < RT; ++rt) {
+      const int r = wr0 + rt * kWR + l % 16;
 #pragma unroll
-    for (int j = 0; j < QPT; ++j) {
-      const int gi = tid + j * NT;
-      const int r = gi / GPR, grp = gi % GPR;
-      *reinterpret_cast<u32x4*>(&sQ[k_off<D>(r, grp)]) = r < rows ? qv[j] : u32x4{0u, 0u, 0u, 0u};
+      for (int kc = 0; kc < KC; ++kc) {
+        qf[rt][kc] = q_at(m0 + min(r, rows - 1), kc);
+        if (r >= rows) qf[rt][kc] = zero;
+        else if (a.scale_log2 < 0.f) qf[rt][kc] = neg(qf[rt][kc]);
+      }
     }
-    if (nx > 0 && tid < kWR * GPR)
-      *reinterpret_cast<u32x4*>(&sQx[k_off<D>(tid / GPR, tid % GPR)]) = tid / GPR < nx ? qx : u32x4{0u, 0u, 0u, 0u};
+    if (EXTRA) {  // the first step's barrier publishes them
+      for (int i = tid; i < kWR * GPR; i += NT) {
+        const int r = i / GPR, m = m0 + kMT + min(r, nx - 1), t = m / a.G, g = m % a.G;
+        const u32x4 v =
+            *reinterpret_cast<const u32x4*>(a.q + (((int64_t)b * a.T + t) * a.Hq + hk * a.G + g) * D + (i % GPR) * 8);
+        *reinterpret_cast<u32x4*>(&sQx[k_off<D>(r, i % GPR)]) =
+            r < nx ? v ^ (a.scale_log2 < 0.f ? 0x80008000u : 0u) : u32x4{0u, 0u, 0u, 0u};
+      }
+    }
   }
 
-  auto stage_step = [&]() {
-#pragma unroll
-    for (int j = 0; j < NKG; ++j) {
-      const int gi = tid + j * NT;
-      *reinterpret_cast<u32x4*>(&sK[k_off<D>(gi / GPR, gi % GPR)]) = kreg[j];
-      *reinterpret_cast<u32x4*>(&sV[v_off<D>(gi / GPR, gi % GPR)]) = vreg[j];
-    }
-  };
-
-  // o[ct] holds O[row][16 ct + 4 (l / 16) + e] of this lane's query row 16 w + l % 16
-  f32x4 o[CT];
-#pragma unroll
-  for (int ct = 0; ct < CT; ++ct) o[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_run = 0.f;
+  // o[rt][ct] holds O[row][16 ct + 4 (l / 16) + e] of this lane's query row of tile rt
+  f32x4 o[RT][CT];
+  f32x4 ox[EXTRA ? XC : 1];  // the extra rows' column tiles [XC w, XC (w + 1))
+  float m_run[ST], l_run[ST];
   // the keys the lane's row sees are exactly [0, klim): the whole prefix, then the block keys its mask
   // allows (a prefix of the block for the causal rows, all of it for the others)
-  int klim;
-  {
-    const int t = (m0 + w * kWR + (l % 16)) / a.G;
+  int klim[ST];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) o[rt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < (EXTRA ? XC : 1); ++c) ox[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int rt = 0; rt < ST; ++rt) {
+    m_run[rt] = -INFINITY;
+    l_run[rt] = 0.f;
+    const int r = rt < RT ? wr0 + rt * kWR + l % 16 : kMT + min(l % 16, max(nx, 1) - 1);
+    const int t = (m0 + r) / a.G;
     const bool all = a.mask_mode == 1 || (a.mask_mode == 2 && t >= a.n_clean);
-    klim = all ? nk : min(nk, prefix + t + 1);
+    klim[rt] = all ? nk : min(nk, prefix + t + 1);
   }
   const int g4 = 4 * (l / 16);
+  const float scale_log2 = fabsf(a.scale_log2);
 
-  // ---- mask, scale and online softmax of one step's scores sc (keys 16 kt + g4 + e of the lane's row, which
-  // sees the keys below lim) against the row's running max m and sum lsum; returns the probabilities as the
-  // B fragments of the two 32-key blocks in pb and the rescale factor of the row's O. The mask applies only
-  // on steps that reach the block keys or the cache end (uniform)
-  auto softmax_step = [&](f32x4 (&sc)[4], int key0, int lim, float& m, float& lsum, u32x4 (&pb)[2]) {
+  // ---- online softmax of one step's raw scores sc (keys 16 kt + g4 + e of the lane's row, which sees the keys
+  // below lim) against the row's running max m (log2 units) and the lane's own part of the row sum, lsum; leaves the
+  // probabilities as the B fragments of the two 32-key blocks in pb. The mask applies only on steps that reach the
+  // block keys or the cache end (uniform); the exchange between a row's four lanes and `rescale` (of the row's O)
+  // run only when a score passes the max. A max that moves only when passed by 2^8 saves most of the moves (205 instead of
+  // 227 us on 64 ragged sequences, 62 instead of 67 on a 512-row chunk), but the largest probabilities are then no longer
+  // just below 1, where bf16 is finest: 2.5 % more error against 64 bits.
+  auto softmax_step = [&](f32x4 (&sc)[4], int key0, int lim, float& m, float& lsum, u32x4 (&pb)[2], auto&& rescale) {
     const bool edge = key0 + kKB > prefix || key0 + kKB > nk;
-#pragma unroll
-    for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sc[kt][e] *= a.scale_log2;
     if (edge) {
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt)
@@ -273,179 +326,162 @@ __global__ __launch_bounds__(kNW* kWave) void attn_partial_kernel(AttnArgs a) {
     float mx = fmaxf(fmaxf(sc[0][0], sc[0][1]), fmaxf(sc[0][2], sc[0][3]));
 #pragma unroll
     for (int kt = 1; kt < 4; ++kt) mx = fmaxf(mx, fmaxf(fmaxf(sc[kt][0], sc[kt][1]), fmaxf(sc[kt][2], sc[kt][3])));
-    mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
-    const float m_new = fmaxf(m, mx);
-    const float m_use = m_new == -INFINITY ? 0.f : m_new;
-    const float alpha = exp2_hw(m - m_use);
-    m = m_new;
-    float ps = 0.f;
+    mx *= scale_log2;
+    if (__ballot(mx > m)) {
+      const float m_new = fmaxf(m, row_max(mx));
+      const float alpha = m_new > m ? exp2_hw(m - m_new) : 1.f;
+      m = m_new;
+      lsum *= alpha;
+      rescale(alpha);
+    }
+    const float m_use = m == -INFINITY ? 0.f : m;
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
       float p[8];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        p[e] = exp2_hw(sc[2 * kk][e] - m_use);
-        p[4 + e] = exp2_hw(sc[2 * kk + 1][e] - m_use);
+        p[e] = fmaf(sc[2 * kk][e], scale_log2, -m_use);
+        p[4 + e] = fmaf(sc[2 * kk + 1][e], scale_log2, -m_use);
+      }
+      if (edge && scale_log2 == 0.f) {  // 0 x -inf
+#pragma unroll
+        for (int e = 0; e < 8; ++e) p[e] = sc[2 * kk + e / 4][e % 4] == -INFINITY ? -INFINITY : p[e];
       }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) ps += p[e];
+      for (int e = 0; e < 8; ++e) {
+        p[e] = exp2_hw(p[e]);
+        lsum += p[e];
+      }
       pb[kk] = u32x4{f2bf2(p[0], p[1]), f2bf2(p[2], p[3]), f2bf2(p[4], p[5]), f2bf2(p[6], p[7])};
     }
-    ps += __shfl_xor(ps, 16, kWave);
-    ps += __shfl_xor(ps, 32, kWave);
-    lsum = lsum * alpha + ps;
-    return alpha;
   };
 
-  // the extra rows: this wave's key tile and column half, its running max / sum over the keys of that tile,
-  // its O^T column tiles, and the keys the lanes' rows see
-  const int ktx = w % 4, dh = w / 4;
-  f32x4 ox[XH];
+  const FragAt<D> at(l);
+  uint32_t vx[EXTRA ? XC : 1];  // FragAt::v of the wave's extra column tiles
+  if (EXTRA) {
 #pragma unroll
-  for (int j = 0; j < XH; ++j) ox[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float mx_run = -INFINITY, lx_run = 0.f;
-  int klim_x = 0;
-  if (nx > 0) {
-    const int t = (m0 + kMT + min(l % 16, nx - 1)) / a.G;
-    const bool all = a.mask_mode == 1 || (a.mask_mode == 2 && t >= a.n_clean);
-    klim_x = all ? nk : min(nk, prefix + t + 1);
+    for (int c = 0; c < XC; ++c)
+      vx[EXTRA ? c : 0] = 2 * (v_off<D>(4 * (l / 16) + (l % 16) / 4, w * XC + c) + 4 * (l % 4));
   }
-  // one step of the extra rows: sx = S^T of key tile ktx (keys 16 ktx + g4 + e of the lane's row)
-  auto extra_step = [&](f32x4 sx, int key0) {
-    const bool edge = key0 + kKB > prefix || key0 + kKB > nk;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      sx[e] *= a.scale_log2;
-      if (edge) sx[e] = key0 + 16 * ktx + g4 + e < klim_x ? sx[e] : -INFINITY;
-    }
-    float mx = fmaxf(fmaxf(sx[0], sx[1]), fmaxf(sx[2], sx[3]));
-    mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
-    const float m_new = fmaxf(mx_run, mx);
-    const float m_use = m_new == -INFINITY ? 0.f : m_new;
-    const float alpha = exp2_hw(mx_run - m_use);
-    mx_run = m_new;
-    float p[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) p[e] = exp2_hw(sx[e] - m_use);
-    float ps = (p[0] + p[1]) + (p[2] + p[3]);
-    ps += __shfl_xor(ps, 16, kWave);
-    ps += __shfl_xor(ps, 32, kWave);
-    lx_run = lx_run * alpha + ps;
-    if (__ballot(alpha != 1.f)) {
-#pragma unroll
-      for (int j = 0; j < XH; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) ox[j][e] *= alpha;
-    }
-    const s16x4 pf = __builtin_bit_cast(s16x4, u32x2{f2bf2(p[0], p[1]), f2bf2(p[2], p[3])});
-    // V^T row (dh XH + j) 16 + l % 16, keys 16 ktx + g4 .. + 3
-#pragma unroll
-    for (int j = 0; j < XH; ++j) {
-      const s16x4 vf = vt_frag4<D>(sV, 16 * ktx, (dh * XH + j) * 16, l);
-      ox[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vf, pf, ox[j], 0, 0, 0);
-    }
-  };
 
-  for (int kb = kb0; kb < kb1; ++kb) {
-    const int key0 = kb * kKB;
-    __syncthreads();  // the previous step's tiles are consumed
-    stage_step();
-    __syncthreads();
-    if (kb + 1 < kb1) load_step(kb + 1);  // in flight during this step's MFMAs
-    // a wave with no row of the tile (a last tile of fewer rows) only helps stage the keys: its fragment
-    // reads and MFMAs would be on padding (wave-uniform; no barrier inside)
-    if (w * kWR >= rows) continue;
-    // ---- S^T = K Q^T: keys 16 kt + 4 (l / 16) + e of this lane's query row (4 key tiles), and key tile ktx
-    // of the extra rows
-    f32x4 sacc[4], sx = f32x4{0.f, 0.f, 0.f, 0.f};
+  // a wave with no row of the tile (a last tile of fewer rows) only loads keys: its fragment
+  // reads and MFMAs would be on padding
+  if (!EXTRA && wr0 >= rows) {
+    for (int kb = kb0; kb < kb1; ++kb) {
+      step_barrier();
+      if (kb + 1 < kb1) load_step(kb + 1, (kb - kb0 + 1) & 1);
+    }
+    return;
+  }
+  auto step = [&](int kb, bool last) {
+    const int key0 = kb * kKB, buf = (kb - kb0) & 1;
+    step_barrier();  // this step's tiles are in, the previous step's are consumed
+    if (!last) load_step(kb + 1, buf ^ 1);  // in flight during this step's MFMAs
+    const uint32_t tk = lds_addr(&sKV[0][0][0]) + (uint32_t)buf * (4 * TILE), tv = tk + 2 * TILE;
+    FragAt<D> fk = at;  // this step's K and V addresses
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt) sacc[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < 2; ++i) fk.k[i] += tk;
+#pragma unroll
+    for (int u = 0; u < FragAt<D>::VU; ++u) fk.v[u] += tv;
+    // ---- S^T = K Q^T: keys 16 kt + 4 (l / 16) + e of this lane's query rows (4 key tiles)
+    f32x4 sacc[ST][4];
+#pragma unroll
+    for (int rt = 0; rt < ST; ++rt)
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt) sacc[rt][kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // fragments are read two k-chunks ahead; the scheduling barriers keep the compiler from hoisting more of
+    // them than there are registers
+    bf16x8 kf[3][4], xf[3];
+    auto read_k = [&](int kc) {
+      if (EXTRA) xf[kc % 3] = at.row(lds_addr(sQx), 0, kc);
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt) kf[kc % 3][kt] = fk.row(0, kt * 16, kc);
+    };
+    read_k(0);
+    if (KC > 1) read_k(1);
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc) {
-      const bf16x8 qf = as_bf16x8(*reinterpret_cast<const u32x4*>(&sQ[k_off<D>(w * kWR + (l % 16), kc * 4 + l / 16)]));
-      bf16x8 kfx = qf;
+      if (kc + 2 < KC) read_k(kc + 2);
 #pragma unroll
-      for (int kt = 0; kt < 4; ++kt) {
-        const bf16x8 kf =
-            as_bf16x8(*reinterpret_cast<const u32x4*>(&sK[k_off<D>(kt * 16 + (l % 16), kc * 4 + l / 16)]));
-        sacc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf, sacc[kt], 0, 0, 0);
-        if (kt == ktx) kfx = kf;
-      }
-      if (nx > 0) {  // block-uniform
-        const bf16x8 qxf = as_bf16x8(*reinterpret_cast<const u32x4*>(&sQx[k_off<D>(l % 16, kc * 4 + l / 16)]));
-        sx = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kfx, qxf, sx, 0, 0, 0);
-      }
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int rt = 0; rt < ST; ++rt)
+          sacc[rt][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[kc % 3][kt], rt < RT ? qf[rt < RT ? rt : 0][kc] : xf[kc % 3],
+                                                                 sacc[rt][kt], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    u32x4 pb[2];
-    const float alpha = softmax_step(sacc, key0, klim, m_run, l_run, pb);
-    // rescale O only when some row's running max moved (rare once the max settles)
-    if (__ballot(alpha != 1.f)) {
+    // V^T fragments, groups of four column tiles, two groups ahead (the first two before the softmax)
+    constexpr int VG = CT / 4, NV = (kKB / 32) * VG;  // groups per 32 keys, in all
+    bf16x8 vf[3][4];
+    auto read_v = [&](int i) {
+      const int kk = i / VG;
 #pragma unroll
-      for (int ct = 0; ct < CT; ++ct)
+      for (int c = 0; c < 4; ++c) {
+        const int ct = (i % VG) * 4 + c;
+        const s16x4 v0 = fk.col(0, 32 * kk, ct), v1 = fk.col(0, 32 * kk + 16, ct);
+        const u32x2 w0 = __builtin_bit_cast(u32x2, v0), w1 = __builtin_bit_cast(u32x2, v1);
+        vf[i % 3][c] = as_bf16x8(u32x4{w0.x, w0.y, w1.x, w1.y});
+      }
+    };
+    read_v(0);
+    read_v(1);
+    __builtin_amdgcn_sched_barrier(0);
+    u32x4 pb[ST][2];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[ct][e] *= alpha;
+    for (int rt = 0; rt < ST; ++rt) {
+      softmax_step(sacc[rt], key0, klim[rt], m_run[rt], l_run[rt], pb[rt], [&](float alpha) {
+        if (rt < RT) {
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[rt < RT ? rt : 0][ct][e] *= alpha;
+        } else {
+#pragma unroll
+          for (int c = 0; c < (EXTRA ? XC : 1); ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ox[c][e] *= alpha;
+        }
+      });
     }
     // ---- O^T += V^T P^T (V^T fragments by transposed LDS reads, in the slot order of the probabilities:
     // keys 32 kk + g4 .. + 3, then 32 kk + 16 + g4 .. + 3)
 #pragma unroll
-    for (int kk = 0; kk < kKB / 32; ++kk) {
-      const bf16x8 pf = as_bf16x8(pb[kk]);
+    for (int i = 0; i < NV; ++i) {
+      if (i + 2 < NV) read_v(i + 2);
 #pragma unroll
-      for (int ct = 0; ct < CT; ++ct) {
-        const s16x4 v0 = vt_frag4<D>(sV, 32 * kk, ct * 16, l), v1 = vt_frag4<D>(sV, 32 * kk + 16, ct * 16, l);
-        const u32x2 w0 = __builtin_bit_cast(u32x2, v0), w1 = __builtin_bit_cast(u32x2, v1);
-        const bf16x8 vf = as_bf16x8(u32x4{w0.x, w0.y, w1.x, w1.y});
-        o[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf, o[ct], 0, 0, 0);
-      }
-    }
-    if (nx > 0) extra_step(sx, key0);
-  }
-  if (nx > 0) {
-    // merge the extra rows' four key-tile states of each column half into its first wave (w % 4 == 0), in
-    // key-tile order; the K / V tiles and Q are no longer read, and sQ holds the other waves' O^T tiles
-    __syncthreads();
-    f32x4* xo = reinterpret_cast<f32x4*>(sQ);  // [column half][key tile 1..3][XH][lane]
-    static_assert(2 * 3 * XH * kWave * 16 <= kMT * D * 2, "the merge's O^T tiles fit in sQ");
-    if (ktx > 0) {
+      for (int c = 0; c < 4; ++c)
 #pragma unroll
-      for (int j = 0; j < XH; ++j) xo[((dh * 3 + ktx - 1) * XH + j) * kWave + l] = ox[j];
-    }
-    if (l < kWR) {
-      sXm[w][l] = mx_run;
-      sXl[w][l] = lx_run;
-    }
-    __syncthreads();
-    if (ktx == 0) {
-      const int rr = l % 16;
-      float mm = mx_run;
-#pragma unroll
-      for (int k = 1; k < 4; ++k) mm = fmaxf(mm, sXm[dh * 4 + k][rr]);
-      const float m_use = mm == -INFINITY ? 0.f : mm;
-      const float e0 = exp2_hw(mx_run - m_use);
-      float ls = lx_run * e0;
-#pragma unroll
-      for (int j = 0; j < XH; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) ox[j][e] *= e0;
-#pragma unroll
-      for (int k = 1; k < 4; ++k) {
-        const float ek = exp2_hw(sXm[dh * 4 + k][rr] - m_use);
-        ls += ek * sXl[dh * 4 + k][rr];
-#pragma unroll
-        for (int j = 0; j < XH; ++j) {
-          const f32x4 v = xo[((dh * 3 + k - 1) * XH + j) * kWave + l];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) ox[j][e] += ek * v[e];
+        for (int rt = 0; rt < RT; ++rt) {
+          const int ct = (i % VG) * 4 + c;
+          o[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[i % 3][c], as_bf16x8(pb[rt][i / VG]), o[rt][ct], 0, 0, 0);
         }
-      }
-      mx_run = mm;
-      lx_run = ls;
+      __builtin_amdgcn_sched_barrier(0);
     }
+    if (EXTRA) {
+#pragma unroll
+      for (int kk = 0; kk < kKB / 32; ++kk)
+#pragma unroll
+        for (int c = 0; c < (EXTRA ? XC : 1); ++c) {
+          const u32x2 w0 = __builtin_bit_cast(
+              u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(tv + vx[c] + (uint32_t)(32 * kk * D * 2))));
+          const u32x2 w1 = __builtin_bit_cast(
+              u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(tv + vx[c] + (uint32_t)((32 * kk + 16) * D * 2))));
+          ox[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(u32x4{w0.x, w0.y, w1.x, w1.y}), as_bf16x8(pb[ST - 1][kk]),
+                                                          ox[c], 0, 0, 0);
+        }
+    }
+  };
+  // the last step, which loads nothing, apart: a conditional load in the loop left O's 128 registers moving
+  // between its blocks
+  for (int kb = kb0; kb + 1 < kb1; ++kb) step(kb, false);
+  step(kb1 - 1, true);
+#pragma unroll
+  for (int rt = 0; rt < ST; ++rt) {  // the rows' sums
+    l_run[rt] += __shfl_xor(l_run[rt], 16, kWave);
+    l_run[rt] += __shfl_xor(l_run[rt], 32, kWave);
   }
-  const int r = w * kWR + (l % 16), rx = kMT + (l % 16);  // the lane's row and extra row of the tile
-  const bool own = r < rows, extra = ktx == 0 && l % 16 < nx;
+  const int rx = kMT + (l % 16);  // the lane's extra row of the tile
+  const bool extra = EXTRA && l % 16 < nx;
   if (a.S == 1) {
     // ---- the only split: O / l, rounded to bf16, then the gate, exactly as the combine computes it
     auto emit = [&](int rr, float lsum, const f32x4& v, int ct) {
@@ -467,13 +503,16 @@ __global__ __launch_bounds__(kNW* kWave) void attn_partial_kernel(AttnArgs a) {
                              : a.out + (((int64_t)b * a.T + t) * a.Hq + hq) * D + c;
       *reinterpret_cast<u32x2*>(dst) = u32x2{f2bf2(y[0], y[1]), f2bf2(y[2], y[3])};
     };
-    if (own) {
 #pragma unroll
-      for (int ct = 0; ct < CT; ++ct) emit(r, l_run, o[ct], ct);
+    for (int rt = 0; rt < RT; ++rt) {
+      const int r = wr0 + rt * kWR + (l % 16);
+      if (r >= min(rows, kMT)) continue;
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) emit(r, l_run[rt], o[rt][ct], ct);
     }
     if (extra) {
 #pragma unroll
-      for (int j = 0; j < XH; ++j) emit(rx, lx_run, ox[j], dh * XH + j);
+      for (int c = 0; c < (EXTRA ? XC : 1); ++c) emit(rx, l_run[ST - 1], ox[c], w * XC + c);
     }
     return;
   }
@@ -483,20 +522,23 @@ __global__ __launch_bounds__(kNW* kWave) void attn_partial_kernel(AttnArgs a) {
   auto park = [&](int rr, const f32x4& v, int ct) {
     *reinterpret_cast<u32x2*>(&op[(int64_t)rr * D + ct * 16 + g4]) = u32x2{f2bf2(v[0], v[1]), f2bf2(v[2], v[3])};
   };
-  if (own) {
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct) park(r, o[ct], ct);
+  for (int rt = 0; rt < RT; ++rt) {
+    const int r = wr0 + rt * kWR + (l % 16);
+    if (r >= min(rows, kMT)) continue;
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) park(r, o[rt][ct], ct);
     if (l < 16) {
-      a.mpart[pbase * kMTX + r] = m_run;
-      a.lpart[pbase * kMTX + r] = l_run;
+      a.mpart[pbase * kMTX + r] = m_run[rt];
+      a.lpart[pbase * kMTX + r] = l_run[rt];
     }
   }
   if (extra) {
 #pragma unroll
-    for (int j = 0; j < XH; ++j) park(rx, ox[j], dh * XH + j);
+    for (int c = 0; c < (EXTRA ? XC : 1); ++c) park(rx, ox[c], w * XC + c);
     if (w == 0 && l < 16) {
-      a.mpart[pbase * kMTX + rx] = mx_run;
-      a.lpart[pbase * kMTX + rx] = lx_run;
+      a.mpart[pbase * kMTX + rx] = m_run[ST - 1];
+      a.lpart[pbase * kMTX + rx] = l_run[ST - 1];
     }
   }
 }
@@ -800,11 +842,19 @@ int attn_canvas_run(const uint16_t* q, const uint16_t* k_cache, const uint16_t* 
              (int)G,      (int)Lmax,       (int)S,           (int)QT,    mask_mode, (int)n_clean, scale * kLog2e, gate,
              gate_row_stride, gate_head_stride, out,         frag ? 1 : 0};
   const dim3 grid((unsigned)slots);
+  // one row tile per wave where that covers the query rows
+  const bool one = T * G <= kNW * kWR;
+  const bool extra = T * G > QT * kMT;
+#define TRIDA_ATTN_PARTIAL(DD)                                                                                   \
+  if (one) hipLaunchKernelGGL((attn_partial_kernel<DD, 1, false>), grid, dim3(kNW * kWave), 0, st, a);           \
+  else if (extra) hipLaunchKernelGGL((attn_partial_kernel<DD, 2, true>), grid, dim3(kNW * kWave), 0, st, a);     \
+  else hipLaunchKernelGGL((attn_partial_kernel<DD, 2, false>), grid, dim3(kNW * kWave), 0, st, a);
   switch (D) {
-    case 64: hipLaunchKernelGGL(attn_partial_kernel<64>, grid, dim3(kNW * kWave), 0, st, a); break;
-    case 128: hipLaunchKernelGGL(attn_partial_kernel<128>, grid, dim3(kNW * kWave), 0, st, a); break;
-    default: hipLaunchKernelGGL(attn_partial_kernel<256>, grid, dim3(kNW * kWave), 0, st, a); break;
+    case 64: TRIDA_ATTN_PARTIAL(64) break;
+    case 128: TRIDA_ATTN_PARTIAL(128) break;
+    default: TRIDA_ATTN_PARTIAL(256) break;
   }
+#undef TRIDA_ATTN_PARTIAL
   int rc = launch_status("attn_canvas/partial");
   if (rc || S == 1) return rc;  // one split: the partial kernel wrote the output
   CombineArgs c{opart, mpart, lpart, gate, out, (int)T, (int)Hq, (int)Hkv, (int)G, (int)D, (int)S, (int)QT,

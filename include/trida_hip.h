@@ -538,6 +538,21 @@ int64_t trida_ws_frag_elems(int64_t K);
 int trida_ws_frag(const uint16_t* X, int64_t x_row_stride, int64_t M, int64_t K, uint16_t* Xf, void* stream);
 int trida_wsgemm_ex(const uint16_t* X, int64_t x_row_stride, const float* ss, float eps, const uint16_t* Wp, int64_t M,
                     int64_t N, int64_t K, int epilogue, void* out, int64_t out_row_stride, int flags, void* stream);
+/* The projections of mid-size row counts (49 <= M <= 512: a small batch's canvases, a prefill chunk) over the same
+ * shuffled weights: Y = X W^T with epilogue 0 (bf16 out [M][N]), 1 (fp32 partial planes [kg][M][N], kg =
+ * trida_wsgemm_mid_plan) or 2 (SwiGLU, bf16 out [M][N / 2]); ss (epilogues 0 and 2, or NULL): the RMSNorm of
+ * trida_wsgemm_norm, X the raw residual rows. N % 16 == 0, K % 32 == 0, any K. X holds trida_ws_mid_elems(M, K) bf16
+ * (16-byte aligned) in the fragment order of trida_ws_frag_elems with ceil(M / 16) row tiles per k-step instead of 3 (the
+ * rows past M are not read into any result); out is row-major (16-byte aligned), or, with TRIDA_WS_OUT_FRAG
+ * (epilogues 0 and 2), in that order for the next product. trida_residual_mid adds the bf16 rows r to h in place and leaves
+ * the sums of squares (ss, as trida_residual_parts) and h in that order. No counterpart in the reference (its
+ * projections are framework matmuls). */
+int64_t trida_ws_mid_elems(int64_t M, int64_t K);
+int trida_residual_mid(uint16_t* h, int64_t h_row_stride, const uint16_t* r, int64_t r_row_stride, int64_t rows,
+                       int64_t dim, float* ss, uint16_t* h_frag, void* stream);
+int trida_wsgemm_mid_plan(int64_t M, int64_t N, int64_t K, int epilogue, int32_t* kgroups);
+int trida_wsgemm_mid(const uint16_t* X, const float* ss, float eps, const uint16_t* Wp, int64_t M, int64_t N, int64_t K,
+                     int epilogue, void* out, int64_t out_row_stride, int flags, void* stream);
 int trida_residual_parts_frag(uint16_t* h, int64_t h_row_stride, const float* parts, int64_t n_parts,
                               int64_t plane_stride, int64_t rows, int64_t dim, float* ss, uint16_t* h_frag,
                               void* stream);

@@ -51,6 +51,10 @@ SIGNATURES = {
     "trida_wsgemm_plan": (C.c_int, [I64, I64, C.c_int, P]),
     "trida_wsgemm": (C.c_int, [P, I64, P, I64, I64, I64, C.c_int, P, I64, P]),
     "trida_wsgemm_norm": (C.c_int, [P, I64, P, F32, P, I64, I64, I64, C.c_int, P, I64, P]),
+    "trida_wsgemm_mid_plan": (C.c_int, [I64, I64, I64, C.c_int, P]),
+    "trida_ws_mid_elems": (I64, [I64, I64]),
+    "trida_residual_mid": (C.c_int, [P, I64, P, I64, I64, I64, P, P, P]),
+    "trida_wsgemm_mid": (C.c_int, [P, P, F32, P, I64, I64, I64, C.c_int, P, I64, C.c_int, P]),
     "trida_residual_ss_chunks": (I64, [I64]),
     "trida_residual_parts": (C.c_int, [P, I64, P, I64, I64, I64, I64, P, P]),
     "trida_ws_frag_elems": (I64, [I64]),

@@ -1113,6 +1113,77 @@ def ws_gemm(x: torch.Tensor, wp: torch.Tensor, N: int, out: torch.Tensor, *, epi
     return out
 
 
+WS_MID_M = 512  # rows ws_gemm_mid takes, from WS_MAX_M + 1 on
+
+
+def ws_mid_planes(M: int, N: int, Kd: int) -> int:
+    """Partial planes ws_gemm_mid writes for M rows with WS_PARTS."""
+    kg = ctypes.c_int32(0)
+    rc = _lib.load().trida_wsgemm_mid_plan(M, N, Kd, WS_PARTS, ctypes.byref(kg))
+    _lib.check(rc, "trida_wsgemm_mid_plan")
+    return kg.value
+
+
+def ws_mid_numel(M: int, Kd: int) -> int:
+    """bf16 elements of the fragment order of M rows of K = Kd columns for ws_gemm_mid."""
+    n = int(_lib.load().trida_ws_mid_elems(M, Kd))
+    if n <= 0:
+        raise ValueError(f"ws_mid_numel: need {WS_MAX_M} < M <= {WS_MID_M} and K a multiple of 32")
+    return n
+
+
+def _mid_buf(t: torch.Tensor, M: int, Kd: int, name: str) -> None:
+    _bf16(t, name)
+    if not t.is_contiguous() or t.numel() < ws_mid_numel(M, Kd):
+        raise ValueError(f"{name}: a fragment-order buffer needs {ws_mid_numel(M, Kd)} contiguous bf16 elements")
+
+
+def residual_mid(h: torch.Tensor, r: torch.Tensor, ss: torch.Tensor, h_frag: torch.Tensor) -> None:
+    """h += r in place (bf16 rows [rows, dim], WS_MAX_M < rows <= WS_MID_M), ss [rows, ss_chunks(dim)] fp32 = the
+    per-chunk sums of h^2 and h_frag = h in the fragment order ws_gemm_mid reads."""
+    dev = _need_gpu(h, r, ss, h_frag)
+    _bf16(h, "h")
+    _bf16(r, "r")
+    rows, dim = h.shape
+    if r.shape != h.shape or h.stride(1) != 1 or r.stride(1) != 1:
+        raise ValueError("residual_mid: h and r must be [rows, dim] with contiguous rows")
+    if ss.dtype != torch.float32 or not ss.is_contiguous() or ss.numel() < rows * ss_chunks(dim):
+        raise ValueError("residual_mid: ss must be contiguous fp32 [rows, ss_chunks(dim)]")
+    _mid_buf(h_frag, rows, dim, "h_frag")
+    rc = _lib.load().trida_residual_mid(h.data_ptr(), h.stride(0), r.data_ptr(), r.stride(0), rows, dim, ss.data_ptr(),
+                                        h_frag.data_ptr(), _stream(dev))
+    _lib.check(rc, "trida_residual_mid")
+
+
+def ws_gemm_mid(xf: torch.Tensor, M: int, wp: torch.Tensor, N: int, out: torch.Tensor, *, ss: Optional[torch.Tensor] = None,
+                eps: float = 1e-6, epilogue: int = WS_STORE, out_frag: bool = False) -> int:
+    """ws_gemm_frag for WS_MAX_M < M <= WS_MID_M rows (xf and, with out_frag, out in the fragment order of M rows:
+    ws_mid_numel). Returns the partial planes written (1 unless WS_PARTS)."""
+    dev = _need_gpu(xf, wp, out, ss)
+    Kd = wp.numel() // N
+    if wp.numel() != N * Kd:
+        raise ValueError("ws_gemm_mid: wp must hold N * K elements")
+    _mid_buf(xf, M, Kd, "xf")
+    if ss is not None and (ss.dtype != torch.float32 or not ss.is_contiguous() or ss.numel() < M * ss_chunks(Kd)):
+        raise ValueError("ws_gemm_mid: ss must be contiguous fp32 [M, ss_chunks(K)]")
+    kg, o_st, width = 1, 0, N // 2 if epilogue == WS_SILU else N
+    if epilogue == WS_PARTS:
+        kg = ws_mid_planes(M, N, Kd)
+        if out_frag or out.dtype != torch.float32 or not out.is_contiguous() or out.numel() < kg * M * N:
+            raise ValueError(f"ws_gemm_mid: partial planes need a contiguous fp32 out of >= {kg} x {M} x {N}")
+    elif out_frag:
+        _mid_buf(out, M, width, "out")
+    else:
+        _bf16(out, "out")
+        if out.dim() != 2 or out.shape[0] < M or out.shape[1] < width or out.stride(1) != 1:
+            raise ValueError(f"ws_gemm_mid: out must be [>= {M}, >= {width}] bf16 with contiguous rows")
+        o_st = out.stride(0)
+    rc = _lib.load().trida_wsgemm_mid(xf.data_ptr(), _ptr(ss), eps, wp.data_ptr(), M, N, Kd, epilogue, out.data_ptr(), o_st,
+                                      WS_OUT_FRAG if out_frag else 0, _stream(dev))
+    _lib.check(rc, "trida_wsgemm_mid")
+    return kg
+
+
 def ws_argmax_splits(N: int, Kd: int) -> int:
     """Column splits (one per workgroup) of the argmax epilogue of an [N, K] weight-streaming GEMM."""
     S = int(_lib.load().trida_wsgemm_argmax_splits(N, Kd))

@@ -7,7 +7,8 @@ Mirrors the reference runtime API of inference/zoro-1/mlx/trida_mlx/model.py:
 plus draft(cache, tokens), the block-diffusion denoising pass (MASK rows see the whole block).
 
 Every hot op runs in a gfx950 kernel of libtrida_hip.so (attention, GDN conv/prep/recurrence/readout,
-rollback, norms, SwiGLU, acceptance); the projections, MLP and LM head are torch GEMMs (hipBLASLt).
+rollback, norms, SwiGLU, acceptance); projections, MLP and LM head run on the weight-streaming GEMMs
+for up to 48 rows, the MLP for up to 512, and on torch GEMMs (hipBLASLt) beyond.
 Caches are batched device tensors: KV [A, B, Hkv, Lmax, D] bf16, GDN state [L, B, Hv, Dv, Dk] fp32 and
 conv window [L, B, Kc-1, C] bf16 (A / L = number of attention / GDN layers). Per-sequence lengths and
 RoPE positions live on the device, so every forward of a given (B, T, mode) has fixed launch shapes
@@ -359,7 +360,8 @@ class TridaRuntime:
 
     def _shuffle_weights(self) -> None:
         """A second copy of every decoder projection and of the LM head in the weight-streaming layout
-        (bf16, the same bytes again: 7.4 + 1.27 GB at the 4B shape), for forwards of <= K.WS_MAX_M rows. A projection whose
+        (bf16, the same bytes again: 7.4 + 1.27 GB at the 4B shape), for forwards of <= K.WS_MAX_M rows
+        (the MLP's: <= K.WS_MID_M). A projection whose
         shape the kernel does not take (N % 16, K % 32, or K too long for a whole-K epilogue) keeps the
         hipBLASLt path. When every projection qualifies (and hidden <= 2560), the forward runs fused: the
         RMSNorm in front of a projection moves into its GEMM, with the norm weight folded into the copy's

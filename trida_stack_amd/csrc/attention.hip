@@ -45,12 +45,6 @@ __device__ __forceinline__ float row_max(float x) {
   return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
-template <int CTRL>
-__device__ __forceinline__ float dpp(float x) {
-  // update_dpp with a defined old value and bound_ctrl: folds into the consuming add / max
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, true));
-}
-
 // 2^x with the hardware instruction: exact for the softmax's arguments x <= 0 down to -126, 0 below
 // (where the library exp2f would return a denormal)
 __device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -90,7 +84,8 @@ template <int D>
 __device__ __forceinline__ int v_off(int key, int unit) { return key * D + ((unit ^ vswz<D>(key)) << 4); }
 
 // 64 lanes x 16 bytes from each lane's address to LDS at `lds` (bytes, wave-uniform) + 16 lane, asynchronously: counted by
-// vmcnt, no register written. In asm because the compiler would wait for it before every later LDS read.
+// vmcnt, no register written. In asm because the compiler would wait for it before every later LDS read; nothing else in these
+// kernels uses m0.
 __device__ __forceinline__ void load_lds16(const uint16_t* src, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory", "m0");
 }

@@ -56,7 +56,8 @@ __device__ __forceinline__ int64_t mid_off(int m, int k, int mt) {
 }
 
 // 64 lanes x 16 bytes to LDS at `lds` (bytes, wave-uniform) + 16 lane, asynchronously: counted by vmcnt, no register
-// written. In asm because the compiler would wait for it before every later LDS read.
+// written. In asm because the compiler would wait for it before every later LDS read; nothing else in these
+// kernels uses m0.
 __device__ __forceinline__ void load_lds16(const u32x4* src, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory", "m0");
 }

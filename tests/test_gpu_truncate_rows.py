@@ -88,3 +88,27 @@ def test_draw_unaligned_rows(gpu, V, dtype):
         lo = cdf[i, tok[i] - 1].item() if tok[i] else 0.0
         assert lo - 1e-6 <= u[i].item() < cdf[i, tok[i]].item() + 1e-6
         assert P.view(B * R, V)[i, tok[i]] > 0
+
+
+def offset_rows(gpu, V, off):
+    """Broad rows, every other one with 20 likely tokens, all shifted by `off` (exactly: multiples of 2^-7 below 2^17)."""
+    g = torch.Generator(device=gpu).manual_seed(17)
+    x = torch.randn(8, V, generator=g, device=gpu) * 2
+    at = torch.randint(0, V, (4, 20), generator=g, device=gpu)
+    x[::2].scatter_add_(1, at, torch.rand(4, 20, generator=g, device=gpu) * 8 + 8)
+    return x.mul(128).round().div(128) + off
+
+
+@pytest.mark.parametrize("off", [0.0, 100.0, -1000.0, 1e5])
+@pytest.mark.parametrize("T", [1.0, 0.5, 2.0])
+def test_offset_untruncated(gpu, T, off):
+    """The normaliser does not depend on a shift of the row. y = x / T is exact at these temperatures, so what is left are
+    roundings at random signs: the exponents' (2^-24 |d log2(e)| ln 2, |d| <= 8 where the mass is), exp2's and the
+    fp32 sums of 16 (2^-24 each), 4e-7 for an entry and less by the root of the 5 or more that carry the mass of the broad
+    rows at T = 0.5; the likely tokens' masses are exact to 2^-26."""
+    x = offset_rows(gpu, 248320, off)
+    m, _, zk, st = TK.truncate_stats(x[None], temperature=T)
+    y = (x.double() / T)
+    z = torch.exp(y - y.amax(-1, keepdim=True)).sum(-1)
+    assert (st == 0).all() and (m[0].double() == y.amax(-1)).all()
+    assert ((zk[0] / z - 1).abs() < 2e-7).all(), (zk[0] / z - 1).tolist()

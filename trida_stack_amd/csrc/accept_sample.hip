@@ -300,7 +300,7 @@ struct BinMap {  // the per-row coefficients of the element -> bin / exponent ma
   float tA, tB;       // t = fma(x, tA, tB)
   float nm;           // -mref
   double rt;          // 1 / T
-  float eA, eB;       // exp(d) = exp2(fma(x, eA, eB)) * cold_scale
+  float eA, eL, eB;   // exp(d) = exp2(cold_exp(x)) * cold_scale
   double cold_scale;  // what the rounding of eB took away
   __device__ unsigned bin(float x) const { return bin_of_t(fmaf(x, tA, tB)); }
   // an element's histogram entry: a count of one and its mass relative to its bin's upper edge
@@ -317,11 +317,19 @@ struct BinMap {  // the per-row coefficients of the element -> bin / exponent ma
     tA = -kPerNat * (float)rt;
     tB = kPerNat * (kTop + mref);
     nm = -mref;
-    const double l2e = 1.4426950408889634;
-    eA = (float)(rt * l2e);
+    const double l2e = 1.4426950408889634, s = rt * l2e;
+    // eA: the 16 leading bits of s less one unit of them; eL, the rest, is positive (x = -inf stays -inf) and never tiny
+    eA = __uint_as_float((__float_as_uint((float)s) & 0xffffff00u) - 0x100u);
+    eL = (float)(s - (double)eA);
     eB = (float)(-(double)mref * l2e);
     cold_scale = exp2(-(double)mref * l2e - (double)eB);
   }
+  // log2(e) d + const in two products, the slope log2(e) / T held to 40 bits. With one fp32 slope every exponent was off
+  // by up to 2^-24 |x / T|, the same way for the whole row; with eL at 2^-24 of eA its product, mostly less than half a
+  // unit of the first sum, was rounded away for the whole row alike. As it is, the roundings of a row's entries are
+  // independent. Normaliser error of untruncated rows at T = 1, one slope -> two: 5.6e-8 -> 3e-9 without a
+  // shift, 1.4e-6 -> 3e-9 at logits of about 100, 1.3e-5 -> 5e-9 at 1000; 0.5 to 1 us of 96 per 512 rows.
+  __device__ float cold_exp(float x) const { return fmaf(x, eL, fmaf(x, eA, eB)); }
 };
 
 // Count of j < lim with base + sum_{i<j} e_i < target, e_i = exp(s_i - m) in fp64 (a prefix, since
@@ -669,7 +677,7 @@ __device__ __forceinline__ void stream_segment(const RowView& rv, const TruncArg
     bool hot = x > x_lo;
     if (kHist) {
       mx = fmaxf(mx, x);
-      const float e = __builtin_amdgcn_exp2f(fmaf(x, bm.eA, bm.eB));
+      const float e = __builtin_amdgcn_exp2f(bm.cold_exp(x));
       cold += hot ? 0.f : e;
     } else {
       hot = hot && x < x_hi;
@@ -1107,8 +1115,9 @@ __global__ __launch_bounds__(kT, 4) void truncate_kernel(TruncArgs a) {
     __syncthreads();
     // ---- the streaming pass, kSeg segments: max, histogram down to the floor, collection of a window placed
     // from the sample's histogram and again from the row's own after every segment. Run again without
-    // floors when the boundary turns out to lie below the last one.
-    int w_lo = kNB + 1, w_hi = kNB + 1, w_top = 0, floor_bin = collect ? kNB : 0;
+    // floors when the boundary turns out to lie below the last one. Without truncation only the few entries above the
+    // sample's max, which may carry most of the mass, go to the histogram: its exponents are exact to 2^-26.
+    int w_lo = kNB + 1, w_hi = kNB + 1, w_top = 0, floor_bin = collect ? kNB : (int)(kTop * kPerNat);
     int seen = 0, counted = ns;
     double tail = 0.0;
     bool floors = true;
@@ -1121,8 +1130,7 @@ __global__ __launch_bounds__(kT, 4) void truncate_kernel(TruncArgs a) {
           sh.whi[s] = min(w_hi, floor_bin - 1);
           sh.top[s] = min(w_top, floor_bin);
         }
-        stream_segment<true>(rv, a, bm, s, collect ? below_bin(bm, floor_bin) : INFINITY, 0.f, w_top, w_lo, w_hi, mx, tail,
-                             have);
+        stream_segment<true>(rv, a, bm, s, below_bin(bm, floor_bin), 0.f, w_top, w_lo, w_hi, mx, tail, have);
         ++passes;
         seen += seg_size(rv, s);
         counted = seen;

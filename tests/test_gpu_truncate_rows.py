@@ -112,3 +112,15 @@ def test_offset_untruncated(gpu, T, off):
     z = torch.exp(y - y.amax(-1, keepdim=True)).sum(-1)
     assert (st == 0).all() and (m[0].double() == y.amax(-1)).all()
     assert ((zk[0] / z - 1).abs() < 2e-7).all(), (zk[0] / z - 1).tolist()
+
+
+@pytest.mark.parametrize("off", [0.0, 5e4, -8e4, 1e5])
+def test_offset_restreamed(gpu, off):
+    """Rows whose likely tokens sit in one tile of the last segment, so that the windows of the earlier ones miss the
+    boundary and their segments are streamed again, shifted by up to 10^5."""
+    g = torch.Generator(device=gpu).manual_seed(5)
+    x = torch.randn(8, 30 * TILE, generator=g, device=gpu) * 2
+    at = 19 * TILE + torch.randint(0, TILE, (8, 20), generator=g, device=gpu)
+    x = (x.scatter_add_(1, at, torch.rand(8, 20, generator=g, device=gpu) * 8 + 4) + off).view(1, 8, -1)
+    assert (TK.truncate_stats(x, temperature=1.0, top_p=0.9, want_passes=True)[4] > 4).all()
+    check(x, 1.0, 0, 0.9)

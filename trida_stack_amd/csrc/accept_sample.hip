@@ -616,6 +616,10 @@ __device__ __forceinline__ int seg_size(const RowView& rv, int s) {
 __device__ __forceinline__ float below_bin(const BinMap& bm, int b) {
   return (bm.tB - ((float)b + 0.5f + 1e-6f * fabsf(bm.tB))) / -bm.tA;
 }
+// And above which no element has a bin >= b: bin b's upper edge, by the same margin further up.
+__device__ __forceinline__ float above_bin(const BinMap& bm, int b) {
+  return (bm.tB - ((float)b - 0.5f - 1e-6f * fabsf(bm.tB))) / -bm.tA;
+}
 
 // Streams a segment of the row in the logits' own units: the division by the temperature is folded into
 // the bin / exponent maps, and the exact y = x / T is only formed for the few collected values.
@@ -1222,7 +1226,7 @@ __global__ __launch_bounds__(kT, 4) void truncate_kernel(TruncArgs a) {
         __syncthreads();
         if (tid == 0) sh.n = n2;
         __syncthreads();
-        const float x_lo = below_bin(bm, c_hi + 1), x_hi = c_lo > 1 ? below_bin(bm, c_lo - 2) : INFINITY;
+        const float x_lo = below_bin(bm, c_hi + 1), x_hi = c_lo > 0 ? above_bin(bm, c_lo) : INFINITY;
         double none = 0.0;
         int unused = 0;
         for (int s = 0; s < kSeg; ++s) {
@@ -1233,7 +1237,8 @@ __global__ __launch_bounds__(kT, 4) void truncate_kernel(TruncArgs a) {
         __syncthreads();
         n2 = min(sh.n, kSortCap);
       }
-      if (use_k) {
+      ok = n2 == need;  // exactly the candidates that the histogram counted; else the exact select
+      if (ok && use_k) {
         collected_to_y<kDiv>(n2, a.rt);
         sort_collection(n2);
         const int k = min(a.top_k, n2);
@@ -1245,7 +1250,7 @@ __global__ __launch_bounds__(kT, 4) void truncate_kernel(TruncArgs a) {
           thr = sh.coll[nk - 1];
         }
         zk = mass_at_least(n2, thr, md);
-      } else {
+      } else if (ok) {
         float ytop, ylow;
         n2 = boundary_to_y<kDiv>(bm, n2, B, a.rt, &ytop, &ylow);
         const double base = cum * exp((double)mref - md), target = (double)a.top_p * Z;

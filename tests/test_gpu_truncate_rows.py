@@ -124,3 +124,21 @@ def test_offset_restreamed(gpu, off):
     x = (x.scatter_add_(1, at, torch.rand(8, 20, generator=g, device=gpu) * 8 + 4) + off).view(1, 8, -1)
     assert (TK.truncate_stats(x, temperature=1.0, top_p=0.9, want_passes=True)[4] > 4).all()
     check(x, 1.0, 0, 0.9)
+
+
+@pytest.mark.parametrize("T,k,p", [(1.0, 0, 1.0), (1.0, 0, 0.95), (2.0, 0, 0.9), (0.7, 50, 0.95), (1.0, 4, 1.0)])
+def test_far_rows(gpu, T, k, p):
+    """Rows masked with the type's lowest value but for 20 tokens that the sample does not see (and one more that it may),
+    ties and steps at 10^8, and at T < 1 the whole row at the lowest value (y = -inf: status 2; else all kept)."""
+    V, g = 25 * TILE + 3, torch.Generator(device=gpu).manual_seed(9)
+    x = torch.full((4, V), torch.finfo(torch.float32).min, device=gpu)
+    x[0, 11 * TILE + 1: 11 * TILE + 41: 2] = torch.randn(20, generator=g, device=gpu) * 3
+    x[1, 5::512] = torch.randn(V // 512 + (V % 512 > 5), generator=g, device=gpu) * 3
+    x[2] = 1e8
+    x[2, : V // 3] -= 8.0
+    check(x[:3].view(1, 3, V), T, k, p)
+    m, thr, zk, st = TK.truncate_stats(x[3].view(1, 1, V), temperature=T, top_k=k, top_p=p)
+    assert st.item() == (2 if T < 1 else 0)
+    if T >= 1:
+        y = x[3, 0] / T
+        assert m.item() == y.item() and zk.item() == V and thr.item() in (y.item(), -float("inf"))

@@ -9,8 +9,8 @@
 //       histogram of the values that can matter (the mass of the others, most of the row, stays in
 //       registers) and collects the window's values into LDS, the window being placed anew from the
 //       histogram after each segment. The boundary bin's values settle thr exactly. Segments whose window
-//       missed are streamed again; rows out of the histogram's range (massive ties, |y| large enough to overflow
-//       the sample-relative exponentials) take an exact radix select over the order-preserving keys of
+//       missed are streamed again; rows out of the histogram's range (massive ties, |y| from 2^18
+//       on) take an exact radix select over the order-preserving keys of
 //       y, 8 bits per pass.
 //       Bound by the instructions of 16 waves per CU beside the row's bytes (two rows per CU at a time). 512
 //       rows of 248320, half of them peaked: 290 -> 184 us at T = 0.7, top_p = 0.95 (478 -> 122 at 0.5 / 0.8,
@@ -1064,7 +1064,7 @@ __global__ __launch_bounds__(kT, 4) void truncate_kernel(TruncArgs a) {
   const bool use_k = a.top_k > 0 && a.top_k < V;
   const bool use_p = a.top_p < 1.f;
   const bool collect = use_k || use_p;
-  const bool window = !(a.flags & 1) && V <= kMaxPackedV;
+  bool window = !(a.flags & 1) && V <= kMaxPackedV && a.rt < 0x1p120;  // (1 / T and its multiples fit fp32)
   int passes = 0;  // segments streamed (kSeg = one pass over the row)
 
   float mx = -INFINITY;  // max logit (the banned id excluded)
@@ -1073,11 +1073,11 @@ __global__ __launch_bounds__(kT, 4) void truncate_kernel(TruncArgs a) {
   int B = -1, need = 0;       // the boundary bin and the entries it takes to resolve it
   float mref = 0.f;
   BinMap bm{};
+  const int ns = min(kSample, V);
+  float xs[kSample / kT];
   if (window) {
     // ---- sample: evenly spaced entries; their max is the exponent reference of the pass, their
     // histogram places the first segment's window
-    const int ns = min(kSample, V);
-    float xs[kSample / kT];
     float smax = -INFINITY;
     if (rv.n4 >= kSample) {
       // kT evenly spaced 16-byte vectors of 4 adjacent entries each: a line per 4 entries (entries one
@@ -1101,11 +1101,17 @@ __global__ __launch_bounds__(kT, 4) void truncate_kernel(TruncArgs a) {
         smax = xs[u] < INFINITY ? fmaxf(smax, xs[u]) : smax;
       }
     }
-    for (int j = tid; j <= kNB; j += kT) sh.hist[j] = 0ull;
     smax = block_max(smax);
     mref = smax > -INFINITY ? exact_y<kDiv>(smax, a.rt) : 0.f;
-    if (fabsf(mref) < 0x1p18f) mref = rintf(mref * kPerNat) / kPerNat;  // a whole bin: see BinMap::packed
+    // Past 2^18 an fp32 y no longer tells bins apart (half a bin to a unit), the bin map rounds by whole bins and, for rows
+    // masked with the type's lowest value, overflows: such a row goes to the exact select.
+    window = fabsf(mref) < 0x1p18f;
+  }
+  if (window) {
+    mref = rintf(mref * kPerNat) / kPerNat;  // a whole bin: see BinMap::packed
     bm.set(a.rt, mref);
+    for (int j = tid; j <= kNB; j += kT) sh.hist[j] = 0ull;
+    __syncthreads();
     LaneBins lb;
     if (tid < kWave) lb.init();
     if (collect) {

@@ -142,3 +142,17 @@ def test_far_rows(gpu, T, k, p):
     if T >= 1:
         y = x[3, 0] / T
         assert m.item() == y.item() and zk.item() == V and thr.item() in (y.item(), -float("inf"))
+
+
+@pytest.mark.parametrize("T,p", [(0.7, 0.95), (1.2, 0.98), (1.0, 0.5)])
+def test_boundary_ties(gpu, T, p):
+    """Widened bf16 rows: the value at the boundary has hundreds of copies; and rows of such values each beside its
+    fp32 neighbour (two values of hundreds of copies in a sub-bin)."""
+    g = torch.Generator(device=gpu).manual_seed(21)
+    x = (torch.randn(4, 30 * TILE + 1, generator=g, device=gpu) * 2).bfloat16().float()
+    x[2:] = torch.where(torch.rand(2, x.shape[1], generator=g, device=gpu) < 0.5, x[2:],
+                        torch.nextafter(x[2:], torch.full_like(x[2:], 9.0)))
+    thr = TK.truncate_stats(x[None], temperature=T, top_p=p)[1][0].cpu()
+    y = x.cpu() / torch.tensor(T)
+    assert (((y - thr[:, None]).abs() < 2e-6).sum(-1) > 64).all()  # more than a wave ranks
+    check(x.view(2, 2, -1), T, 0, p)

@@ -962,7 +962,7 @@ __device__ __forceinline__ int boundary_to_y(const BinMap& bm, int n, int B, dou
 // one that crosses tgt, and one wave ranks its few values against each other (a bitonic sort of all of
 // them took a quarter of the kernel's instructions). *mass: the mass of every value >= thr. Masses are summed as
 // integers, 46 bits below ytop's: the result does not depend on the order. False (nothing done to sh.coll) when
-// the sub-bin holds more than a wave's values.
+// the sub-bin holds more than a wave's values that are not all equal.
 __device__ __forceinline__ bool sub_boundary(int n, float ytop, float ylow, double tgt, float* thr, double* mass) {
   const int tid = threadIdx.x;
   unsigned long long* sub = sh.hist;
@@ -1016,16 +1016,26 @@ __device__ __forceinline__ bool sub_boundary(int n, float ytop, float ylow, doub
     return true;
   }
   float* list = sh.queue[0];
+  float lo = INFINITY, hi = -INFINITY;
   for (int j = tid; j < n; j += kT) {
     const float y = sh.coll[j];
     if (sub_of(y) == S) {
+      lo = fminf(lo, y);
+      hi = fmaxf(hi, y);
       const int at = atomicAdd(&sh.n, 1);
       if (at < kWave) list[at] = y;
     }
   }
   __syncthreads();
   const int cnt = sh.n;
-  if (cnt > kWave) return false;
+  if (cnt > kWave) {  // more than a wave's values, unless they are one: rows of widened bf16 logits hold hundreds of each
+    lo = -block_max(-lo);
+    hi = block_max(hi);
+    if (lo != hi) return false;
+    *thr = hi;
+    *mass = (above + (double)sub[S]) * 0x1p-46;
+    return true;
+  }
   if (tid < kWave) {
     const float y = tid < cnt ? list[tid] : -INFINITY;
     const unsigned long long q = tid < cnt ? mass_of(y) : 0ull;

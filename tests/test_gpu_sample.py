@@ -262,3 +262,24 @@ def test_sample_accept_config5_shape(gpu):
     ok = ~ref["tie"]
     assert (n_acc[sel][ok] == ref["n_acc"][ok]).all()
     assert (tok[sel][ok] == ref["token"][ok]).all()
+
+
+@pytest.mark.parametrize("B", [1, 7, 9])
+def test_sample_accept_longest_block(gpu, B):
+    """K = 64, the most drafts: the bonus row is the 65th, one past a wave's lanes, and its status and its draw count
+    like any other row's (the first sequence's bonus row holds a NaN, the last's is all -inf)."""
+    K, V = 64, 300
+    g = torch.Generator(device=DEV).manual_seed(B)
+    drafts = torch.randint(0, V, (B, K), generator=g, device=DEV)
+    p = torch.randn(B, K + 1, V, generator=g, device=DEV)
+    p[:, :K].scatter_(2, drafts[..., None], 20.0)
+    p[:, K, 17] = 30.0
+    want = [0] * B
+    if B > 1:
+        p[-1, K], want[-1] = -float("inf"), 2
+    p[0, K, 5], want[0] = float("nan"), 1
+    q = torch.full((B, K, V), 1.0 / V, device=DEV)
+    n_acc, tok, _, _, st = TK.sample_accept(p, q, drafts, torch.full((B, K), 0.5, device=DEV), torch.rand(B, generator=g, device=DEV),
+                                            temperature=1.0, top_p=0.9)
+    assert n_acc.tolist() == [K] * B and st.tolist() == want
+    assert tok[1:-1].tolist() == [17] * max(B - 2, 0)

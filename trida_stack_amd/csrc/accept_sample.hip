@@ -1719,11 +1719,11 @@ extern "C" int trida_sample_accept(const float* p_logits, int64_t B, int64_t R, 
                 ban_of(ban_id, V), m, thr, zk, st, state, rstatus, NC, chunk, sums, n_acc, token, crop, ratio, status};
 
   // Only rows up to a sequence's first rejection decide anything. Rows 0..G0-1 of every sequence go
-  // first (G0 sized so that this group alone fills the GPU, ~512 blocks); a one-wave scan per
+  // first (G0 sized so that this group alone fills the GPU, ~512 blocks, and a row per lane of the scan); a one-wave scan per
   // sequence then settles the sequences it can, and one more group evaluates all the remaining rows
   // of the rest at once (decided sequences' blocks exit at once), followed by the final scan.
   const int R1 = (int)K + 1;
-  const int G0 = (int)std::min<int64_t>(R1, std::max<int64_t>(8, cdiv(512, B)));
+  const int G0 = (int)std::min<int64_t>({R1, std::max<int64_t>(8, cdiv(512, B)), kWave});
   int r = TRIDA_OK;
   for (int g = 0; g < 2; ++g) {
     const int first = g == 0 ? 0 : G0, cnt = g == 0 ? G0 : R1 - G0;

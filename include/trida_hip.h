@@ -227,7 +227,7 @@ int trida_sample_rows(const float* logits, int64_t rows, int64_t V, int64_t row_
  * not NULL; window_out must not alias window. pre_out [B, T, C] (contiguous, 16-byte aligned, not x)
  * receives a copy of the pre-conv rows x when not NULL: the rows a rollback rebuilds the conv window
  * from (the raw mixed_qkv rows that fused_selfspec_gdn_layer keeps, qwen3_5_diffusion.py:2219).
- * Dk in {32, 64, 128}, Dv % 8 == 0.
+ * Dk in {32, 64, 128}, Dv % 8 == 0; C <= 8192 where B * T >= 512.
  * State-pool and packed forms (each NULL = the contiguous form above), the arguments of the vLLM
  * calls this replaces (causal_conv1d_fn(x, weight, bias, conv_states, cache_indices, query_start_loc),
  * qwen3_5_diffusion.py:2227-2231; fused_selfspec_gdn_layer's conv_bias / win / win_idx / pre_out /

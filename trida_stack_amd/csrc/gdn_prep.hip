@@ -278,7 +278,9 @@ extern "C" int trida_gdn_prep(const uint16_t* x, const uint16_t* window, const u
   // 16, in chunks of equal length: 9.6 -> 7.6 us at 512 rows (4 per block), 12.2 -> 8.3 at 16 x 33 with pre_out. 300
   // rows take 5.3 us one per block, their launch and one memory round trip.
   const bool multi = B * T >= 512;
-  TRIDA_CHECK(!multi || C <= 8 * 256 * 4, TRIDA_ERR_ARG, "gdn_prep: conv_dim %lld above %d", (long long)C, 8 * 256 * 4);
+  // part of the entry point's contract, not of this launch: wider rows are refused here as they always were
+  constexpr int kMaxWideC = 8192;
+  TRIDA_CHECK(!multi || C <= kMaxWideC, TRIDA_ERR_ARG, "gdn_prep: conv_dim %lld above %d", (long long)C, kMaxWideC);
   const int64_t slices = cdiv(C / 8, kNT);
   const int64_t most = multi ? std::max<int64_t>(4, std::min<int64_t>(16, B * T * slices / 1536)) : 1;
   a.chunks = (int)cdiv(T, most);

@@ -156,3 +156,14 @@ def test_boundary_ties(gpu, T, p):
     y = x.cpu() / torch.tensor(T)
     assert (((y - thr[:, None]).abs() < 2e-6).sum(-1) > 64).all()  # more than a wave ranks
     check(x.view(2, 2, -1), T, 0, p)
+
+
+@pytest.mark.parametrize("T,p", [(1.0, 0.95), (0.7, 0.8), (1.2, 0.3)])
+def test_flat_rows(gpu, T, p):
+    """Rows from near-flat to broad: the two bins at the boundary hold from all of the row down to a few thousand values,
+    across the collection's 12288, the 8192 that are sorted and the rule that skips the streaming pass."""
+    g = torch.Generator(device=gpu).manual_seed(31)
+    std = torch.tensor([0.002, 0.05, 0.1, 0.2, 0.25, 0.3, 0.35, 0.4, 0.5, 0.6, 0.8, 1.0], device=gpu) * T
+    x = torch.randn(12, 30 * TILE, generator=g, device=gpu) * std[:, None]
+    x[1, 2::3] = -float("inf")
+    check(x.view(2, 6, -1), T, 0, p)

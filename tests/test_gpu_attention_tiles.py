@@ -44,6 +44,25 @@ def test_extra_rows(gpu, D, rows):
     check(gpu, B, rows, 2, 2, D, [(13 * i) % 90 for i in range(B)], 2)
 
 
+@pytest.mark.parametrize("T", [65, 68, 97])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_extra_rows_of_the_last_tile(gpu, T, splits):
+    """Several query tiles of which the last has extra rows (4 T = 260, 272, 388): the rows before the last tile are bit by
+    bit those of the same sequence alone, whose tiles have no extra rows."""
+    B, G, D = 100, 4, 256
+    g = torch.Generator(device=gpu).manual_seed(T)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=gpu).to(torch.bfloat16)
+    pre = torch.tensor([(13 * i) % 190 for i in range(B)], dtype=torch.int32, device=gpu)
+    q, k, v = rnd(B, T, G, D), rnd(B, 1, 190 + T, D), rnd(B, 1, 190 + T, D)
+    out = K.attn_canvas(q, k, v, pre, mask_mode=0, splits=splits)
+    ref = A.canvas_attention(q[:9].float().cpu(), k[:9].float().cpu(), v[:9].float().cpu(), pre[:9].tolist(), 0, 0)
+    assert rel(out[:9], ref) < TOL
+    n = (4 * T - 1) // 128 - 1  # whole tiles before the last
+    for b in (0, 1, 8, B - 1):
+        one = K.attn_canvas(q[b:b + 1], k[b:b + 1], v[b:b + 1], pre[b:b + 1], mask_mode=0, splits=splits)
+        assert torch.equal(out[b, :32 * n], one[0, :32 * n]) and rel(out[b], one[0]) < TOL
+
+
 @pytest.mark.parametrize("keys", [1, 63, 64, 65, 127, 128, 129, 193])
 @pytest.mark.parametrize("splits", [1, 2, 0])
 def test_key_steps(gpu, keys, splits):

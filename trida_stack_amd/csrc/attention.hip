@@ -126,6 +126,12 @@ struct FragAt {
   }
 };
 
+struct Tile {  // a workgroup's part, block-uniform
+  int b, hk, m0, rows, nx;   // sequence, KV head, first query row, rows, those past kMT
+  int prefix, nk, kb0, kb1;  // keys: the committed ones, all, the split's 64-key steps
+  int64_t pbase;             // the split's slot of the partial results
+};
+
 // Workgroup = (sequence, KV head, query tile of kMT rows, key split); 4 waves, wave w owns RT row tiles of 16: rows
 // [16 RT w, 16 RT (w + 1)) of the tile, their Q as B fragments in registers. Per 64-key step, K and V are staged
 // in one of two LDS buffers while the next step's tiles stream into the other (global_load_lds), and the
@@ -146,7 +152,7 @@ struct FragAt {
 // Extra rows (EXTRA: the last tile's kMT .. kMT + 15): a third row tile of every wave, from the K fragments the wave
 // reads for its own rows (Q from LDS); of their O^T, wave w accumulates the column tiles [XC w, XC (w + 1)).
 template <int D, int RT, bool EXTRA>
-__global__ __launch_bounds__(kNW* kWave, D == 256 ? 1 : 2) void attn_partial_kernel(AttnArgs a) {
+__device__ __forceinline__ void attn_tile(const AttnArgs& a, const Tile& wt, uint16_t (*sKV)[2][kKB * D], uint16_t* sQx) {
   constexpr int KC = D / 32;         // 32-wide k-chunks of the head dim (QK^T)
   constexpr int CT = D / 16;         // 16-column tiles of O
   constexpr int GPR = D / 8;         // 16-byte groups per K row
@@ -156,76 +162,11 @@ __global__ __launch_bounds__(kNW* kWave, D == 256 ? 1 : 2) void attn_partial_ker
   constexpr int ST = RT + (EXTRA ? 1 : 0);  // row tiles that form scores: the extra rows are the last one
   constexpr int XC = CT / kNW;              // column tiles of the extra rows per wave
   constexpr int TILE = kKB * D;
-  // [buffer][K, V] tiles
-  __shared__ __align__(16) uint16_t sKV[2][2][TILE];
-  __shared__ __align__(16) uint16_t sQx[EXTRA ? kWR * D : 8];  // the extra rows' Q, as K
 
   const int tid = threadIdx.x, w = tid / kWave, l = tid % kWave;
-  const int per_pair = a.S * a.QT;                  // workgroups per (sequence, KV head)
-  const int npair = (int)gridDim.x / per_pair, nseq = npair / a.Hkv;
-  int b, hk, s, qt;
-  if (nseq > 1 && nseq <= kMaxLptSeqs && npair % kXcds == 0) {
-    // ragged batches: longest sequences first. Workgroups reach the XCDs round-robin in block order,
-    // so (sequence, KV head) pairs are dealt to the XCDs in descending prefix length, each pair's
-    // workgroups consecutive on one XCD (its query tiles share the keys in that L2); the longest pairs
-    // start in the first wave of workgroups instead of wherever their batch index put them.
-    __shared__ int s_len[kMaxLptSeqs];
-    __shared__ int s_seq;
-    const int x = (int)blockIdx.x % kXcds, j = (int)blockIdx.x / kXcds;
-    const int pr = (j / per_pair) * kXcds + x;  // pair rank
-    const int wi = j % per_pair;
-    qt = wi % a.QT;
-    s = wi / a.QT;
-    hk = pr % a.Hkv;
-    const int r = pr / a.Hkv;  // sequence rank: prefix length descending, batch index ascending
-    for (int c = tid; c < nseq; c += kNW * kWave) s_len[c] = a.prefix[c];
-    __syncthreads();
-    for (int c = tid; c < nseq; c += kNW * kWave) {
-      const int lc = s_len[c];
-      int rank = 0;
-      for (int o = 0; o < nseq; ++o) rank += (s_len[o] > lc) | ((s_len[o] == lc) & (o < c));
-      if (rank == r) s_seq = c;
-    }
-    __syncthreads();
-    b = s_seq;
-  } else {
-    // query tiles of one (split, kv head) read the same keys: innermost, and on one XCD
-    int idx = xcd_major(blockIdx.x, gridDim.x);
-    qt = idx % a.QT;
-    idx /= a.QT;
-    s = idx % a.S;
-    idx /= a.S;
-    hk = idx % a.Hkv;
-    b = idx / a.Hkv;
-  }
-  const int M = a.T * a.G;
-  const int m0 = qt * kMT;
-  // the tile's rows: kMT, or for the last tile all that remain (<= kMTX: nx extra rows past kMT)
-  const int rows = qt == a.QT - 1 ? M - m0 : kMT;
-  const int nx = max(rows - kMT, 0);  // block-uniform
-  // a prefix past the cache capacity (a caller's overlong decode) is clamped so that every key read
-  // stays inside this sequence's [Lmax, D] rows
-  const int prefix = min(max(a.prefix[b], 0), a.Lmax - a.T);
-  const int nk = prefix + a.T;
-  const int nblk = (nk + kKB - 1) / kKB;
-  const int bps = (nblk + a.S - 1) / a.S;
-  const int kb0 = s * bps;
-  // the last query row of the tile bounds the keys any row can see under the causal masks
-  const int t_last = (m0 + rows - 1) / a.G;
-  const int kmax = (a.mask_mode == 1 || (a.mask_mode == 2 && t_last >= a.n_clean)) ? nk : min(nk, prefix + t_last + 1);
-  const int kb1 = min(min(nblk, kb0 + bps), (kmax + kKB - 1) / kKB);
-
-  const int64_t pbase = ((((int64_t)b * a.Hkv + hk) * a.QT + qt) * a.S + s);
-  if (kb0 >= kb1) {
-    // no key of this split is visible to the tile: only the (empty) row stats are written and the
-    // combine skips the split without reading its O (never with one split: its keys start at 0 and every
-    // row sees at least its own)
-    for (int r = tid; r < rows; r += NT) {
-      a.mpart[pbase * kMTX + r] = -INFINITY;
-      a.lpart[pbase * kMTX + r] = 0.f;
-    }
-    return;
-  }
+  const int b = wt.b, hk = wt.hk, m0 = wt.m0, rows = wt.rows, nx = wt.nx;
+  const int prefix = wt.prefix, nk = wt.nk, kb0 = wt.kb0, kb1 = wt.kb1;
+  const int64_t pbase = wt.pbase;
   const uint16_t* kh = a.k_cache + ((int64_t)b * a.Hkv + hk) * a.Lmax * D;
   const uint16_t* vh = a.v_cache + ((int64_t)b * a.Hkv + hk) * a.Lmax * D;
 
@@ -538,6 +479,88 @@ __global__ __launch_bounds__(kNW* kWave, D == 256 ? 1 : 2) void attn_partial_ker
   }
 }
 
+// The launch: no extra rows, extra rows in every tile (the only one of its rows), or in the last of several, of which
+// the others then form none. With the third row tile of zeros scored in all tiles, 64 sequences of 33 rows x 8 heads took 356
+// instead of 344 us at head dim 256 (512-4096 keys), 32 of 67 x 4 177 instead of 171. At 64 and 128 both forms take the
+// same (78, 154-155 us), and one tile in the launch of several is 1-2 % slower (its registers): those take kAll.
+enum ExtraRows { kNone = 0, kAll = 1, kLast = 2 };
+template <int D, int RT, int X>
+__global__ __launch_bounds__(kNW* kWave, D == 256 ? 1 : 2) void attn_partial_kernel(AttnArgs a) {
+  // [buffer][K, V] tiles
+  __shared__ __align__(16) uint16_t sKV[2][2][kKB * D];
+  __shared__ __align__(16) uint16_t sQx[X ? kWR * D : 8];  // the extra rows' Q, as K
+
+  const int tid = threadIdx.x;
+  const int per_pair = a.S * a.QT;                  // workgroups per (sequence, KV head)
+  const int npair = (int)gridDim.x / per_pair, nseq = npair / a.Hkv;
+  int b, hk, s, qt;
+  if (nseq > 1 && nseq <= kMaxLptSeqs && npair % kXcds == 0) {
+    // ragged batches: longest sequences first. Workgroups reach the XCDs round-robin in block order,
+    // so (sequence, KV head) pairs are dealt to the XCDs in descending prefix length, each pair's
+    // workgroups consecutive on one XCD (its query tiles share the keys in that L2); the longest pairs
+    // start in the first wave of workgroups instead of wherever their batch index put them.
+    __shared__ int s_len[kMaxLptSeqs];
+    __shared__ int s_seq;
+    const int x = (int)blockIdx.x % kXcds, j = (int)blockIdx.x / kXcds;
+    const int pr = (j / per_pair) * kXcds + x;  // pair rank
+    const int wi = j % per_pair;
+    qt = wi % a.QT;
+    s = wi / a.QT;
+    hk = pr % a.Hkv;
+    const int r = pr / a.Hkv;  // sequence rank: prefix length descending, batch index ascending
+    for (int c = tid; c < nseq; c += kNW * kWave) s_len[c] = a.prefix[c];
+    __syncthreads();
+    for (int c = tid; c < nseq; c += kNW * kWave) {
+      const int lc = s_len[c];
+      int rank = 0;
+      for (int o = 0; o < nseq; ++o) rank += (s_len[o] > lc) | ((s_len[o] == lc) & (o < c));
+      if (rank == r) s_seq = c;
+    }
+    __syncthreads();
+    b = s_seq;
+  } else {
+    // query tiles of one (split, kv head) read the same keys: innermost, and on one XCD
+    int idx = xcd_major(blockIdx.x, gridDim.x);
+    qt = idx % a.QT;
+    idx /= a.QT;
+    s = idx % a.S;
+    idx /= a.S;
+    hk = idx % a.Hkv;
+    b = idx / a.Hkv;
+  }
+  const int M = a.T * a.G;
+  const int m0 = qt * kMT;
+  // the tile's rows: kMT, or for the last tile all that remain (<= kMTX: nx extra rows past kMT)
+  const int rows = qt == a.QT - 1 ? M - m0 : kMT;
+  const int nx = max(rows - kMT, 0);  // block-uniform
+  // a prefix past the cache capacity (a caller's overlong decode) is clamped so that every key read
+  // stays inside this sequence's [Lmax, D] rows
+  const int prefix = min(max(a.prefix[b], 0), a.Lmax - a.T);
+  const int nk = prefix + a.T;
+  const int nblk = (nk + kKB - 1) / kKB;
+  const int bps = (nblk + a.S - 1) / a.S;
+  const int kb0 = s * bps;
+  // the last query row of the tile bounds the keys any row can see under the causal masks
+  const int t_last = (m0 + rows - 1) / a.G;
+  const int kmax = (a.mask_mode == 1 || (a.mask_mode == 2 && t_last >= a.n_clean)) ? nk : min(nk, prefix + t_last + 1);
+  const int kb1 = min(min(nblk, kb0 + bps), (kmax + kKB - 1) / kKB);
+
+  const int64_t pbase = ((((int64_t)b * a.Hkv + hk) * a.QT + qt) * a.S + s);
+  if (kb0 >= kb1) {
+    // no key of this split is visible to the tile: only the (empty) row stats are written and the
+    // combine skips the split without reading its O (never with one split: its keys start at 0 and every
+    // row sees at least its own)
+    for (int r = tid; r < rows; r += kNW * kWave) {
+      a.mpart[pbase * kMTX + r] = -INFINITY;
+      a.lpart[pbase * kMTX + r] = 0.f;
+    }
+    return;
+  }
+  const Tile wt{b, hk, m0, rows, nx, prefix, nk, kb0, kb1, pbase};
+  if (X == kLast && nx == 0) attn_tile<D, RT, false>(a, wt, sKV, sQx);
+  else attn_tile<D, RT, X != kNone>(a, wt, sKV, sQx);
+}
+
 struct CombineArgs {
   const uint16_t* opart;  // bf16
   const float* mpart;
@@ -841,9 +864,11 @@ int attn_canvas_run(const uint16_t* q, const uint16_t* k_cache, const uint16_t* 
   const bool one = T * G <= kNW * kWR;
   const bool extra = T * G > QT * kMT;
 #define TRIDA_ATTN_PARTIAL(DD)                                                                                   \
-  if (one) hipLaunchKernelGGL((attn_partial_kernel<DD, 1, false>), grid, dim3(kNW * kWave), 0, st, a);           \
-  else if (extra) hipLaunchKernelGGL((attn_partial_kernel<DD, 2, true>), grid, dim3(kNW * kWave), 0, st, a);     \
-  else hipLaunchKernelGGL((attn_partial_kernel<DD, 2, false>), grid, dim3(kNW * kWave), 0, st, a);
+  if (one) hipLaunchKernelGGL((attn_partial_kernel<DD, 1, kNone>), grid, dim3(kNW * kWave), 0, st, a);           \
+  else if (extra && QT > 1)                                                                                      \
+    hipLaunchKernelGGL((attn_partial_kernel<DD, 2, DD == 256 ? kLast : kAll>), grid, dim3(kNW * kWave), 0, st, a); \
+  else if (extra) hipLaunchKernelGGL((attn_partial_kernel<DD, 2, kAll>), grid, dim3(kNW * kWave), 0, st, a);     \
+  else hipLaunchKernelGGL((attn_partial_kernel<DD, 2, kNone>), grid, dim3(kNW * kWave), 0, st, a);
   switch (D) {
     case 64: TRIDA_ATTN_PARTIAL(64) break;
     case 128: TRIDA_ATTN_PARTIAL(128) break;

@@ -64,6 +64,38 @@ def test_products(gpu, M, N, Kd):
             assert torch.equal(unfrag(af, M, N // 2), act)
 
 
+@pytest.mark.parametrize("M", [49, 128, 129, 264, 385, 512])
+def test_wide_plans(gpu, M):
+    """The products of the 4B-shape MLP, whose plans take 3 to 5 column tiles per workgroup (1216 tiles in fives: the
+    last workgroup has one) and split K over up to 6 groups, where the shapes above take 2 tiles and at most 3 groups."""
+    g = torch.Generator(device=gpu).manual_seed(M)
+    N, Kd = 19456, 2560
+    h = torch.randn(M, Kd, generator=g, device=gpu).to(torch.bfloat16)
+    w = (torch.randn(N, Kd, generator=g, device=gpu) * Kd ** -0.5).to(torch.bfloat16)
+    ss, hf, wp = torch.empty(M, K.ss_chunks(Kd), device=gpu), frag(h), K.ws_shuffle(w)
+    K.residual_mid(h, torch.zeros_like(h), ss, torch.empty_like(hf))
+    out = torch.full((M, N + 4), -7.0, dtype=torch.bfloat16, device=gpu)
+    K.ws_gemm_mid(hf, M, wp, N, out[:, :N])
+    assert rel(out[:, :N], h.double() @ w.double().t()) < 2 ** -8 and (out[:, N:] == -7).all()
+    n = h.double() * torch.rsqrt((h.double() ** 2).mean(-1, keepdim=True) + 1e-6)
+    gate, up = (n @ w.double().t()).to(torch.bfloat16).double().split(N // 2, -1)
+    y = torch.nn.functional.silu(gate) * up
+    wq = K.ws_shuffle(w, pair_halves=True)
+    act = torch.full((M, N // 2 + 4), -7.0, dtype=torch.bfloat16, device=gpu)
+    K.ws_gemm_mid(hf, M, wq, N, act[:, :N // 2], ss=ss, epilogue=K.WS_SILU)
+    assert rel(act[:, :N // 2], y) < 2 ** -7 and (act[:, N // 2:] == -7).all()
+    af = torch.empty(K.ws_mid_numel(M, N // 2), dtype=torch.bfloat16, device=gpu)
+    K.ws_gemm_mid(hf, M, wq, N, af, ss=ss, epilogue=K.WS_SILU, out_frag=True)
+    assert torch.equal(unfrag(af, M, N // 2), act[:, :N // 2])
+
+    w2 = (torch.randn(Kd, N // 2, generator=g, device=gpu) * (N // 2) ** -0.5).to(torch.bfloat16)
+    kg = K.ws_mid_planes(M, Kd, N // 2)
+    parts = torch.empty(kg, M, Kd, device=gpu)
+    assert K.ws_gemm_mid(af, M, K.ws_shuffle(w2), Kd, parts, epilogue=K.WS_PARTS) == kg
+    ref = act[:, :N // 2].double() @ w2.double().t()
+    assert rel(parts.double().sum(0), ref) < 2e-6  # fp32 sums of 32 products at a time, at most 9728 / 32 of them
+
+
 @pytest.mark.parametrize("B,T", [(7, 7), (4, 33), (16, 32), (1, 300)])
 @pytest.mark.parametrize("mid", [True, False])
 def test_forward_mlp(gpu, B, T, mid):

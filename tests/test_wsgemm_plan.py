@@ -3,6 +3,7 @@ for the 4B-shape projections and the shapes it rejects."""
 import pytest
 
 from trida_stack_amd import kernels as TK
+from trida_stack_amd.model import HybridConfig, _Scratch
 
 
 @pytest.mark.parametrize("N,K,epi,kg", [
@@ -37,3 +38,14 @@ def test_partial_plans_are_deterministic():
 def test_rejected_plans(N, K, epi):
     with pytest.raises(ValueError):
         TK.ws_plan(N, K, epi)
+
+
+@pytest.mark.parametrize("rows,planes,mid", [(33, 4, False), (64, 4, True), (512, 4, True), (64, 0, False), (513, 0, False)])
+def test_scratch_holds_one_form_of_the_mlp_rows(rows, planes, mid):
+    """The MLP's row buffers: row-major, or (mid-size row counts on the weight-streaming GEMM) in fragment order."""
+    cfg = HybridConfig.tiny(vocab=320)
+    s = _Scratch(cfg, 1, rows, 2, "cpu", ws_parts=planes)
+    for t in (s.gu_p, s.act_p, s.gu, s.act):
+        assert (t is None) == mid
+    for t in (s.hm, s.actm):
+        assert (t is not None) == mid

@@ -204,13 +204,18 @@ class _Scratch:
         self.h = torch.empty(N, h, **bf)
         self.x_p = torch.zeros(Np, h, **bf)
         self.r_p = torch.zeros(Np, h, **bf)
-        self.gu_p = torch.zeros(Np, 2 * cfg.intermediate, **bf)
-        self.act_p = torch.zeros(Np, cfg.intermediate, **bf)
+        # the MLP on the mid-size weight-streaming GEMM (its inputs in fragment order), or row-major
+        mid = ws_parts and N > K.WS_MAX_M
+        self.hm = torch.empty(K.ws_mid_numel(N, h), **bf) if mid else None
+        self.actm = torch.empty(K.ws_mid_numel(N, cfg.intermediate), **bf) if mid else None
+        self.gu_p = None if mid else torch.zeros(Np, 2 * cfg.intermediate, **bf)
+        self.act_p = None if mid else torch.zeros(Np, cfg.intermediate, **bf)
         self.proj_p = torch.zeros(Np, W_in, **bf)
         self.qkv_p = torch.zeros(Np, W_qkv, **bf)
         self.o_att_p = torch.zeros(Np, cfg.n_heads * cfg.head_dim, **bf)
         self.yn_p = torch.zeros(Np, cfg.lin_v_heads * cfg.lin_v_dim, **bf)
-        self.x, self.r, self.gu, self.act = self.x_p[:N], self.r_p[:N], self.gu_p[:N], self.act_p[:N]
+        self.x, self.r = self.x_p[:N], self.r_p[:N]
+        self.gu, self.act = (None, None) if mid else (self.gu_p[:N], self.act_p[:N])
         self.proj = self.proj_p[:N].view(B, T, W_in)
         self.qkv = self.qkv_p[:N].view(B, T, W_qkv)
         self.o_att = self.o_att_p[:N].view(B, T, cfg.n_heads, cfg.head_dim)
@@ -227,10 +232,6 @@ class _Scratch:
         self.pre_rec = torch.empty(n_gdn, B, T, cfg.conv_dim, **bf)
         # split-K partial planes of the weight-streaming GEMM ([kg, N, hidden] fp32), when it runs here
         self.parts = torch.empty(max(1, ws_parts) * N * h, **f32) if ws_parts else None
-        # the MLP on the mid-size weight-streaming GEMM: its inputs in fragment order
-        mid = ws_parts and N > K.WS_MAX_M
-        self.hm = torch.empty(K.ws_mid_numel(N, h), **bf) if mid else None
-        self.actm = torch.empty(K.ws_mid_numel(N, cfg.intermediate), **bf) if mid else None
         self.ss = torch.empty(N, (h + 255) // 256, **f32) if ws_parts else None  # per-chunk sums of h^2
         # the fused forward's GEMM inputs in the weight-streaming GEMM's fragment order (h, the SwiGLU
         # output, the gated-norm output), written by their producers

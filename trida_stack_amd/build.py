@@ -32,7 +32,8 @@ HIPCC_FLAGS = [
 
 # attention.hip: MFMA accumulators in the ordinary registers. Its kernels of head dim 256 hold more than 256 registers,
 # for which the compiler would keep the accumulators in the accumulation half and move them at every rescale and
-# loop edge (about 400 moves a step, a third of its instructions).
+# loop edge (about 400 moves a step, a third of its instructions). An option of the compiler's own: one that does not
+# know it builds the file without.
 FILE_FLAGS = {"attention": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 
@@ -45,8 +46,12 @@ def hipcc() -> str:
 
 def _compile(src: Path) -> Path:
     obj = OBJ / (src.stem + ".o")
-    cmd = [hipcc(), *HIPCC_FLAGS, *FILE_FLAGS.get(src.stem, []), "-c", str(src), "-o", str(obj)]
-    r = subprocess.run(cmd, capture_output=True, text=True)
+    extra = FILE_FLAGS.get(src.stem, [])
+    cmd = [hipcc(), *HIPCC_FLAGS, "-c", str(src), "-o", str(obj)]
+    r = subprocess.run([*cmd, *extra], capture_output=True, text=True)
+    if r.returncode != 0 and extra and "Unknown command line argument" in r.stderr:
+        print(f"[trida] {src.name}: this compiler does not know {' '.join(extra)}; built without (slower kernels)", flush=True)
+        r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src.name}:\n{r.stdout}\n{r.stderr}")
     return obj

@@ -63,6 +63,21 @@ def test_extra_rows_of_the_last_tile(gpu, T, splits):
         assert torch.equal(out[b, :32 * n], one[0, :32 * n]) and rel(out[b], one[0]) < TOL
 
 
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("B,rows", [(2, 1), (2, 17), (2, 63), (2, 65), (2, 127), (140, 129), (140, 144), (140, 260)])
+def test_gate_of_the_only_split(gpu, D, B, rows):
+    """The gated output of one split against the ungated one: bf16(o) sigmoid(gate), rounded to bf16 (2^-8; the hardware
+    exponential is within 2^-20)."""
+    g = torch.Generator(device=gpu).manual_seed(rows + D)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=gpu).to(torch.bfloat16)
+    q, k, v, gate = rnd(B, rows, 2, D), rnd(B, 2, 300, D), rnd(B, 2, 300, D), rnd(B, rows, 2, 2 * D)[..., D:]
+    pre = torch.tensor([(7 * i) % 40 for i in range(B)], dtype=torch.int32, device=gpu)
+    plain = K.attn_canvas(q, k, v, pre, mask_mode=0, splits=1)
+    out = K.attn_canvas(q, k, v, pre, mask_mode=0, splits=1, gate=gate)
+    want = plain.double() * torch.sigmoid(gate.double())
+    assert ((out.double() - want).abs() <= want.abs() * 2 ** -8).all()
+
+
 @pytest.mark.parametrize("keys", [1, 63, 64, 65, 127, 128, 129, 193])
 @pytest.mark.parametrize("splits", [1, 2, 0])
 def test_key_steps(gpu, keys, splits):

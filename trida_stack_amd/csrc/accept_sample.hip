@@ -13,10 +13,11 @@
 //       on) take an exact radix select over the order-preserving keys of
 //       y, 8 bits per pass.
 //       Bound by the instructions of 16 waves per CU beside the row's bytes (two rows per CU at a time). 512
-//       rows of 248320, half of them peaked: 290 -> 184 us at T = 0.7, top_p = 0.95 (478 -> 122 at 0.5 / 0.8,
-//       259 -> 242 at 1.2 / 0.98, where two thirds of a row are kept and the boundary moves with each late
-//       token), 230 -> 122 with top_k = 50, 118 -> 98 (5.2 TB/s) untruncated; rows of 248319, which scalar loads
-//       served: 588 -> 169.
+//       rows of 248320, half of them peaked, against every element in the histogram: 231 -> 182 us at T = 0.7,
+//       top_p = 0.95 (413 -> 123 at 0.5 / 0.8, 257 -> 250 at 1.2 / 0.98, where two thirds of a row are kept and the
+//       boundary moves with each late token), 181 -> 113 with top_k = 50, 111 -> 94 (5.4 TB/s) untruncated; rows
+//       of 248319, which scalar loads served: 572 -> 176. Widened bf16 rows take the same (177 at 0.7 / 0.95;
+//       in the draft pass, behind the launch that has just written them, 210).
 //   resid_sums (grid NC x B): every block re-derives its sequence's accepted length from the drafted
 //       tokens' ratios P_i(d_i) / q_i(d_i), then sums the correction weights max(0, P_a - q_a) (P_K
 //       when every draft is accepted) and P_a over its chunk of the vocabulary, in fp64.

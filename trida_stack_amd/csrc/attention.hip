@@ -137,18 +137,19 @@ struct Tile {  // a workgroup's part, block-uniform
 // in one of two LDS buffers while the next step's tiles stream into the other (global_load_lds), and the
 // wave forms the transposed products S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_16x16x32_bf16, so lane l holds
 // 16 scores and 256 / 4 output values of one query row (l % 16) of each tile: the online softmax of a row is
-// the lane's own, completed across its four lane groups by two xor exchanges, and its probabilities are, as
+// the lane's own, completed across its four lane groups by two lane swaps, and its probabilities are, as
 // computed, the B operand of the product with V (a 32-key block takes slots 8 g + j = keys 32 kk + 4 g + j
 // and 32 kk + 16 + 4 g + j - 4, which is where the two key tiles' accumulators put them). O is rescaled only
 // when a row's running max moved. Writes the unnormalised O, the row max (log2 domain) and the row sum of its split.
 // Each K and V fragment read feeds RT products: what bounds a step is LDS reads (each wave reads both tiles, 64
 // KB at D = 256), so 32 rows per wave halve them against 16. RT = 1 serves tiles of <= 64 rows, whose waves
 // would otherwise be idle.
-// Against 8 waves of 16 rows, tiles staged through registers between two barriers and Q in LDS: 64 sequences of 33
-// rows and 512-4096 keys 253 -> 215 us (head dim 256; 128: 134 -> 99), a 512-row chunk behind 3584 keys 82 -> 67,
-// 33 rows over 8192 keys 34 -> 31, 64 sequences of one row 117 -> 111 (5.4 TB/s of keys). A step of 32 rows per
-// wave takes about 3 us of MFMA, LDS reads and softmax one after the other, as 2 x 64 KB of tiles leave room for
-// one workgroup per CU.
+// A call with its combine, against 8 waves of 16 rows, tiles staged through registers between two barriers and Q in LDS: 64
+// sequences of 33 rows and 512-4096 keys 232 -> 205 us (head dim 256, nothing cached; 128: 131 -> 113.5), a 512-row
+// chunk behind 3584 keys 73 -> 60.5, 33 rows over 8192 keys 32.9 -> 29.4, 50 sequences of 7 rows and 300 keys
+// 39.2 -> 35.1. With one to three key steps per workgroup and more than one split it is up to 1 % slower (2 x 32
+// rows over 5738 keys 38.7 -> 39.2). A step of 32 rows per wave takes about 3 us of MFMA, LDS reads and softmax one after
+// the other, as 2 x 64 KB of tiles leave room for one workgroup per CU.
 // Extra rows (EXTRA: the last tile's kMT .. kMT + 15): a third row tile of every wave, from the K fragments the wave
 // reads for its own rows (Q from LDS); of their O^T, wave w accumulates the column tiles [XC w, XC (w + 1)).
 template <int D, int RT, bool EXTRA>
@@ -806,12 +807,14 @@ __global__ __launch_bounds__(kC2T) void attn_combine2_kernel(CombineArgs a) {
 }
 
 // Splits per (sequence, KV head, query tile): as many as keep the grid within one workgroup per CU
-// (a workgroup holds a CU's LDS), at least one key block each. Measured at batch 1 (33 canvas rows,
-// 16 / 4 heads, d 256): 2200 keys 30.0 -> 25 us, 8192 keys 54.2 -> 40 us against splits of >= 4 key
-// blocks; a grid just past the CU count (33 splits) runs a ragged second round and is slower.
+// (a workgroup holds a CU's LDS), at least one key block each. Measured at batch 1 (33 canvas rows, 16 / 4 heads,
+// d 256, us by splits, 32 being the plan): 8192 keys 8: 54.6, 16: 36.9, 28: 29.4, 32: 29.9; 2048 keys 8: 26.5, 21: 21.7,
+// 32: 22.5; a grid just past the CU count (36 splits) runs a ragged second round, 44.4 at 8192 keys.
 // When the query tiles alone fill the CUs (a batch of sequences), two splits per tile, so that the
 // longest sequences of a ragged batch are not one workgroup's serial walk over their keys (64 sequences
-// of 512-4096 keys, 32 rows x 4 heads: 245 -> 201 us).
+// of 512-4096 keys, 33 rows x 4 heads, one query tile each: 1 split 245 us, 2: 189, 3: 212, 4: 226; 128 of them are even,
+// 329 and 364). Between half of the CUs and all of them the first rule leaves one split, which is not the
+// best there: 48 such sequences 232 us, with two splits 157; 24 of two tiles each 163, with two 102.
 constexpr int64_t kCUs = 256;
 int64_t plan_splits(int64_t B, int64_t Hkv, int64_t QT, int64_t max_keys, int64_t splits) {
   if (splits > 0) return splits;
@@ -825,8 +828,10 @@ int64_t plan_splits(int64_t B, int64_t Hkv, int64_t QT, int64_t max_keys, int64_
 
 // Query tiles of M rows per (sequence, KV head): kMT rows each. A last one of <= 16 rows joins the tile
 // before it as its extra rows when its own workgroups would not fit beside the others on the CUs (a batch
-// of sequences; 64 x 33 rows x 4 heads, 512-4096 keys: 277 -> 243 us). Where they fit (batch 1) they run
-// on otherwise idle CUs and the extra rows' work would only lengthen the full tile's (23.1 -> 25.5 us).
+// of sequences; 64 x 33 rows x 4 heads, 512-4096 keys: 237 us apart, 188 joined). Where they fit (batch 1) they run
+// on otherwise idle CUs and the extra rows' work would only lengthen the full tile's (8192 keys 29.9 us apart, 32.0 joined;
+// 2048 keys 22.5 and 24.8; 2 sequences 26.7 and 30.5). The two meet before the CUs are full: 8 sequences 49.2 and 45.8,
+// 16 89 and 77, and 32 130 and 120 with three splits (135 with the planned two).
 int64_t query_tiles(int64_t B, int64_t Hkv, int64_t M) {
   const int64_t qt = cdiv(M, kMT);
   return qt > 1 && M - (qt - 1) * kMT <= kWR && B * Hkv * qt > kCUs ? qt - 1 : qt;

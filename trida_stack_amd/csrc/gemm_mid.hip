@@ -13,8 +13,11 @@
 //     26 instead of 15. The producers write that order (trida_residual_mid, this kernel's SwiGLU epilogue);
 //   - fragment by fragment the products are v_mfma_f32_16x16x32_bf16 with W as the A operand, as in gemm.hip.
 // K may be split over kg groups of workgroups that write partial planes (summed in plane order by the consumer).
-// Bound by the L2 -> CU traffic: every workgroup reads all of X (17 TB/s in all; M x K x 2 bytes x N / (16 T)
-// workgroups) besides the weights from HBM. Measured beside the library's GEMM (gate / up with its SwiGLU pass;
+// Bound at 64 rows by the weights' stream (4.2 TB/s), from 264 rows on by the workgroup's own k-steps. Gate / up with X
+// read from one k-step only, W from one 4 KB only, both: 64 rows 23.9 -> 23.5, 14.3, 13.8 us; 264 rows 42.7 -> 38.9,
+// 31.6, 30.1; 512 rows 59.1 -> 55.7, 49.8, 47.5. What is left at 264 rows is 0.34 us a k-step: 0.2 of matrix instructions
+// on the busiest SIMD, the rest LDS reads of the fragments (each wave reads all of the stage) that they do not cover;
+// the memory latency of W adds a third. Every workgroup reads all of X from L2 (in all, with W, 10-12 TB/s). Measured beside the library's GEMM (gate / up with its SwiGLU pass;
 // MI355X, cold weights): gate / up 19456 x 2560 30 -> 25 us at 64 rows, 42 -> 32 at 132, 51 -> 43 at 264, 64 -> 59 at
 // 512; down 2560 x 9728 25 -> 14, 27 -> 20, 34 -> 25, 50 -> 35. Whole-K bf16 outputs of narrower weights are
 // no faster (8224 x 2560: 15 -> 13, 19 -> 17, 22 -> 23, 32 -> 35), so those projections stay with the library.
@@ -195,7 +198,9 @@ struct Plan {
 // Column tiles per workgroup and K splits by the cycles of the busiest CU: per k-step the largest of the matrix work
 // (the row tiles of one SIMD's two waves, 16 cycles a tile), the loads (64 B per cycle of X and weights) and the
 // LDS reads (8 waves, 128 B per cycle); 6000 for a workgroup's first loads and its epilogue; partial planes at the
-// memory's 2 KB per cycle, written and read.
+// memory's 2 KB per cycle, written and read. Against T = 2..5 and 1 to 8 splits at 64, 132, 264 and 512 rows the plan is
+// the fastest or within 1 us of it: gate / up at 264 rows T = 2: 69, 3: 55, 4: 63, 5: 41 us (planned); down there T = 3 in
+// 4 splits 27.1, 4 in 6 25.5 (planned), 5 in 8 24.9, 4 in 1 82; at 132 rows 3 in 4 20.4 (planned), 4 in 6 19.5.
 Plan plan_mid(int64_t M, int64_t N, int64_t K, int epi) {
   const int64_t tiles = N / 16, nsteps = K / 32, mt = cdiv(M, 16);
   Plan best{0, 0};
